@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "fpv2_common.h"
 
 namespace fpv2 {
@@ -30,6 +32,18 @@ int check_launch(const char* kernel) {
   if (e != hipSuccess) return fail(FPV2_ERR_LAUNCH, "%s: launch failed: %s", kernel, hipGetErrorString(e));
   g_error[0] = '\0';
   return FPV2_OK;
+}
+
+int cu_count() {
+  static std::atomic<int> cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 }  // namespace fpv2

@@ -103,6 +103,11 @@ __device__ __forceinline__ float quad_sum(float x) {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 
+// Balanced walk: the workgroups of the head that walk a (tile, row chunk).
+struct BalCut {
+  int first, last;
+};
+
 struct AttnArgs {
   const uint16_t* q;
   const uint16_t* k;
@@ -130,8 +135,13 @@ struct AttnArgs {
   // writing unnormalised partials (O, l) and their scale m (the partial is
   // (O, l) * 2^m in the common scale of exp2(logit)) for merge_split_kernel.
   int split_tiles, nseg, seg_steps;
-  float* ws_o;    // [item][seg][RW rows][D]
-  float* ws_ml;   // [item][seg][RW rows][2]: m, l
+  float* ws_o;    // [partial][RW rows][D]; split: partial = item * nseg + seg
+  float* ws_ml;   // [partial][RW rows][2]: m, l
+  // Balanced walk (bal_wgs > 0): bal_wgs workgroups per KV head walk the
+  // head's last split_tiles tiles in parts (see bal_part); partial =
+  // h * bal_wgs + g.
+  int bal_wgs;
+  BalCut* cuts;   // [h * split_tiles * nchunk + item]
 };
 
 // Workgroup barrier for data written to LDS by ds_write: it waits for this
@@ -146,6 +156,113 @@ __device__ __forceinline__ V pick(bool c, V x, V y) {
 }
 __device__ __forceinline__ int clampi(int x, int lo, int hi) {
   return x < lo ? lo : (x > hi ? hi : x);
+}
+
+// ---------------------------------------------------------------------------
+// Balanced walk: bal_wgs workgroups per KV head (as many as the chip holds at
+// once) walk the head's (tile, row chunk) items in parts.  An item whose walk
+// has `len` steps, taken from its list counts, becomes ceil(len / quantum)
+// equal parts, one workgroup each; the quantum is the smallest (in steps of
+// an eighth) for which the head's parts do not exceed its workgroups, and at
+// least kBalPart steps: a part costs its set-up and its partial's traffic,
+// about 10 steps (with 48, 55-step walks of 64 tiles at D = 256 took 83 us
+// instead of 58).  The head's items must not exceed its workgroups.
+//   Why: a tile walked by one workgroup leaves most of the chip idle in calls
+// of few tiles.  64 tiles (one KV head, 2048 queries) on 512 workgroup slots,
+// D = 128, 510 steps a tile: 336 us whole, 81 us in parts; two of a 20001-key
+// dense tail's tiles per head at D = 256, in fixed 128-step segments 167 us,
+// in parts 45 us.  (Workgroups that take several parts in a loop, so that
+// every share is equal, were 10-17 % slower per step: the loop's registers
+// spill.)  merge_balanced_kernel adds the
+// partials of the items of several parts.  Every workgroup computes the same
+// plan from the head's counts, so nothing is exchanged and the result is
+// deterministic.
+// ---------------------------------------------------------------------------
+constexpr int kBalPart = 32;
+
+template <bool CORR>
+__device__ __forceinline__ int bal_len(const AttnArgs& a, int h, int item) {
+  const int row = h * a.Nt + a.Nt - 1 - item / a.nchunk;
+  int len = clampi(a.counts[row], 0, a.Nb) * ((a.bk + 31) / 32);
+  if (CORR) len += (clampi(a.pcounts[row], 0, a.Nb) + 31) / 32;
+  return max(len, 1);
+}
+
+// The part of workgroup g of head h: its item and steps [lo, hi), and whether
+// it is all of the item's walk.  False: no part.  `lds`: 64 ints, free again
+// on return; all THREADS threads of the workgroup call it.
+template <bool CORR, int THREADS>
+__device__ __forceinline__ bool bal_part(const AttnArgs& a, int h, int g, int* lds, int& item, int& lo, int& hi, bool& all) {
+  constexpr int NW = THREADS / 64;
+  constexpr int PER = 4;  // items per thread held in registers; more are read again
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = a.split_tiles * a.nchunk;
+  const int per = (n + THREADS - 1) / THREADS;
+  const int i0 = min(n, tid * per), i1 = min(n, i0 + per);
+  int keep[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) keep[j] = i0 + j < i1 ? bal_len<CORR>(a, h, i0 + j) : 0;
+  auto len_of = [&](int i) {
+    int len = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) len = i - i0 == j ? keep[j] : len;
+    return i - i0 < PER ? len : bal_len<CORR>(a, h, i);
+  };
+  // sum of v over the workgroup, and over the threads before this one
+  auto scan = [&](int v, int& before) {
+    int incl = v;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+      const int u = __shfl_up(incl, o);
+      if (lane >= o) incl += u;
+    }
+    __syncthreads();  // the previous scan's values have been read
+    if (lane == 63) lds[wave] = incl;
+    __syncthreads();
+    int total = 0;
+    before = incl - v;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      before += w < wave ? lds[w] : 0;
+      total += lds[w];
+    }
+    return __builtin_amdgcn_readfirstlane(total);
+  };
+  int sum = 0, before = 0;
+  for (int i = i0; i < i1; ++i) sum += len_of(i);
+  const int total = scan(sum, before);
+  int quantum = max(kBalPart, (total + a.bal_wgs - 1) / a.bal_wgs), parts = 0;
+  for (;;) {
+    parts = 0;
+    for (int i = i0; i < i1; ++i) parts += (len_of(i) + quantum - 1) / quantum;
+    if (scan(parts, before) <= a.bal_wgs) break;
+    quantum += quantum / 8;  // (one part per item fits: it ends)
+  }
+  // the thread whose items hold part g
+  __syncthreads();
+  if (tid == 0) lds[0] = -1;
+  __syncthreads();
+  if (before <= g && g < before + parts) {
+    int at = before, i = i0, k = 0, len = 0;
+    for (;; ++i) {
+      len = len_of(i);
+      k = (len + quantum - 1) / quantum;
+      if (g < at + k) break;
+      at += k;
+    }
+    const int step = (len + k - 1) / k;
+    lds[0] = i;
+    lds[1] = (g - at) * step;
+    lds[2] = g - at == k - 1 ? 0x7fffffff : (g - at + 1) * step;
+    if (g == at) a.cuts[static_cast<int64_t>(h) * n + i] = BalCut{g, g + k - 1};
+  }
+  __syncthreads();
+  item = __builtin_amdgcn_readfirstlane(lds[0]);
+  lo = __builtin_amdgcn_readfirstlane(lds[1]);
+  hi = __builtin_amdgcn_readfirstlane(lds[2]);
+  all = lo == 0 && hi == 0x7fffffff;
+  __syncthreads();
+  return item >= 0;
 }
 
 // LDS geometry of one K or V sub-tile: BN rows of ROWB bytes (D elements
@@ -192,10 +309,10 @@ struct Step {
 // softmax work is not repeated.  Each accumulates its half of O from both
 // halves of P.  This keeps D = 256 at two waves per SIMD within 256
 // registers.
-// SEG: the launch of the split tiles' segments (every workgroup is one
-// segment of one split tile), instantiated apart so that the whole-tile
-// kernel's code carries nothing of it.
-template <typename T, int D, bool CORR, int WAVES, int NST, int DS = 1, bool SEG = false>
+// FLEX: workgroups that walk parts of tiles (the split dense tail, the
+// balanced walk), instantiated apart so that the whole-tile kernel's code
+// carries nothing of it.
+template <typename T, int D, bool CORR, int WAVES, int NST, int DS = 1, bool FLEX = false>
 __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void sparse_attn_kernel(AttnArgs a) {
   using GM = Geom<D>;
   constexpr int RT = 2;  // 16-row query tiles per wave (32 rows)
@@ -226,22 +343,37 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
   __shared__ __align__(1024) uint8_t smem[NST * GM::STAGE + (DS == 2 ? WAVES * 4096 : 0)];
   uint8_t* const xbuf = smem + NST * GM::STAGE;
 
+  // ---- workgroup -> (KV head, tile, row chunk); latest tiles first ----
+  // The KV head is in the low bits.  Whole tiles: [0, Nt - split_tiles).
+  // FLEX: a part of one of the tiles [Nt - split_tiles, Nt).
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
   const int l16 = lane & 15;
   const int grp = lane >> 4;  // 16-lane group: keys 4*grp.. of each key tile
-
-  // ---- workgroup -> (KV head, tile, row chunk); latest tiles first ----
-  // Whole tiles: [0, Nt - split_tiles).  Segments (SEG): seg of the split
-  // tiles [Nt - split_tiles, Nt).  The KV head is in the low bits.
   const int bid = blockIdx.x;
   const int h = bid % a.Hkv;
-  int rest = bid / a.Hkv;
-  const int seg = SEG ? rest % a.nseg : -1;
-  if constexpr (SEG) rest /= a.nseg;
-  const int chunk = rest % a.nchunk;
-  const int t = (SEG ? a.Nt : a.Nt - a.split_tiles) - 1 - rest / a.nchunk;
+  int item = bid / a.Hkv;   // (tile, row chunk), latest tile first
+  int part_lo = 0;          // the part of the tile's walk: [part_lo, part_hi)
+  int part_hi = 0x7fffffff;
+  int partial = -1;         // the partial to write (-1: the output)
+  if constexpr (FLEX) {
+    if (a.bal_wgs > 0) {
+      const int g = item;
+      bool all;
+      if (!bal_part<CORR, WAVES * 64>(a, h, g, reinterpret_cast<int*>(smem), item, part_lo, part_hi, all)) return;
+      if (!all) partial = h * a.bal_wgs + g;
+    } else {
+      const int seg = item % a.nseg;
+      item /= a.nseg;
+      part_lo = seg * a.seg_steps;
+      part_hi = part_lo + a.seg_steps;
+      // (merge_split_kernel's order: head, tile, chunk, segment)
+      partial = ((h * a.split_tiles + a.split_tiles - 1 - item / a.nchunk) * a.nchunk + item % a.nchunk) * a.nseg + seg;
+    }
+  }
+  const int chunk = item % a.nchunk;
+  const int t = a.Nt - 1 - (FLEX ? 0 : a.split_tiles) - item / a.nchunk;
   const int abs_first = a.offset + t * a.tq;
   const int last_local = min((t + 1) * a.tq, a.Lq);
   const int abs_last = a.offset + last_local - 1;
@@ -388,16 +520,15 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
   auto load_window = [&](int base) {  // raw entry of step base + lane
     return static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(idr, ((base + lane) / subs) * 4, 0, 0));
   };
-  // A workgroup walks steps [s_lo, s_hi): all of the tile's, or a
-  // segment's seg_steps of them.
-  const int s_lo = SEG ? min(seg * a.seg_steps, n_steps) : 0;
-  const int s_hi = SEG ? min(s_lo + a.seg_steps, n_steps) : n_steps;
+  // A workgroup walks steps [s_lo, s_hi): all of the tile's, or a part.
+  const int s_lo = FLEX ? min(part_lo, n_steps) : 0;
+  const int s_hi = FLEX ? min(part_hi, n_steps) : n_steps;
   // The window holding step s: the first window's entries come from id_lane
   // (its steps cover at most the first 64 entries), later ones are loaded.
   int win_next = 0;
   auto start_windows = [&](int s) {
-    win_base = SEG ? (s / 64) * 64 : 0;
-    if (!SEG || win_base == 0) {
+    win_base = FLEX ? (s / 64) * 64 : 0;
+    if (!FLEX || win_base == 0) {
       window_entry(lane, __builtin_amdgcn_ds_bpermute((lane / subs) * 4, id_lane));
     } else {
       const int li = (win_base + lane) / subs;  // < li_end when the step is < n_sel
@@ -654,7 +785,7 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
   // stage in the instruction's immediate offset: the XOR terms touch
   // address bits 4-7 only, which a stage offset (a multiple of the stage
   // size) leaves alone.
-  constexpr bool kImm = !KSPLIT && !SEG;
+  constexpr bool kImm = !KSPLIT;
   static_assert(!kImm || (NST - 1) * GM::STAGE + 16 * ROWB < 65536, "ds offset field is 16 bits");
   uint32_t kx[KSQ], vx[DT];
   if constexpr (kImm) {
@@ -1177,14 +1308,14 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
     // taken as exp2(S), their relative weight 2^shift (kernel.py:349-351);
     // O / l is unchanged by the common factor.  (A rescale inside the walk
     // would make the compiler move O between register ranges every slice.)
-    // (every segment of a tile with correction steps takes the rescale,
-    // so that their partials share one scale)
-    walk_end = SEG ? min(s_hi, n_sel) : n_sel;
+    // (every part of a tile with correction steps takes the rescale, so
+    // that their partials share one scale)
+    walk_end = FLEX ? min(s_hi, n_sel) : n_sel;
     // (the two walks are instantiated for their kinds of steps, except with
     // the D split, whose kernel measured 1 % slower with the second walk)
     using KindExact = std::integral_constant<int, KSPLIT ? 0 : 1>;
     using KindCorr = std::integral_constant<int, KSPLIT ? 0 : 2>;
-    if (!SEG || walk_it < walk_end) run_walk(False{}, KindExact{}, False{});
+    if (!FLEX || walk_it < walk_end) run_walk(False{}, KindExact{}, False{});
     if (n_corr > 0) {
       __syncthreads();  // every wave is done with the ring before it is refilled
 #pragma unroll
@@ -1193,27 +1324,29 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) scale_in_place(o[dt][rt], a.inv_bk);
       }
-      walk_it = SEG ? max(s_lo, n_sel) : n_sel;
+      walk_it = FLEX ? max(s_lo, n_sel) : n_sel;
       walk_end = s_hi;
-      if (!SEG || walk_it < walk_end) run_walk(False{}, KindCorr{}, False{});
+      if (!FLEX || walk_it < walk_end) run_walk(False{}, KindCorr{}, False{});
     }
-  } else if constexpr (CORR && !SEG && !KSPLIT) {
-    // float16 with correction: the exact steps, then the correction steps,
-    // whose slices keep the reference the first exact slice fixed.  (A
-    // tile of the hook always selects a block, the largest energy passing
-    // any alpha <= 1; a tile whose lists, given through the C ABI, select
-    // none has no fixed reference and takes the online walk below.)
-    walk_end = n_sel;
-    run_walk(False{}, std::integral_constant<int, 1>{}, False{});
-    if (n_corr > 0) {
-      __syncthreads();  // every wave is done with the ring before it is refilled
-      walk_it = n_sel;
-      walk_end = s_hi;
-      run_walk(False{}, std::integral_constant<int, 2>{}, True{});
+  } else if (!FLEX || kFree || s_lo == 0) {
+    if constexpr (CORR && !KSPLIT) {
+      // float16 with correction: the exact steps, then the correction steps,
+      // whose slices keep the reference the first exact slice fixed.  (A
+      // tile of the hook always selects a block, the largest energy passing
+      // any alpha <= 1; a tile whose lists, given through the C ABI, select
+      // none has no fixed reference and takes the online walk below.)
+      walk_end = FLEX ? min(s_hi, n_sel) : n_sel;
+      run_walk(False{}, std::integral_constant<int, 1>{}, False{});
+      if (FLEX ? s_hi > n_sel : n_corr > 0) {
+        __syncthreads();  // every wave is done with the ring before it is refilled
+        walk_it = n_sel;
+        walk_end = s_hi;
+        run_walk(False{}, std::integral_constant<int, 2>{}, True{});
+      }
+    } else {
+      // (without correction every step is exact)
+      run_walk(False{}, std::integral_constant<int, CORR ? 0 : 1>{}, False{});
     }
-  } else {
-    // (without correction every step is exact)
-    run_walk(False{}, std::integral_constant<int, CORR ? 0 : 1>{}, False{});
   }
   row_sums();
   bool bad = false;
@@ -1228,7 +1361,12 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
     const float l = l_tot[rt];
     bad = bad || (row_valid[rt] && !(l >= 0x1p-60f && l <= 0x1p64f && fin));
   }
-  if constexpr (CORR && !kFree && !SEG && !KSPLIT) bad = bad || n_sel == 0;  // (see the walks above)
+  if constexpr (CORR && !kFree && !KSPLIT) bad = bad || n_sel == 0;  // (see the walks above)
+  // A float16 part that does not start its tile has no first slice to fix a
+  // reference by (the tile's first block is the sink; a later part may meet
+  // logits far above its own first slice, and would walk twice): one online
+  // walk.
+  if constexpr (FLEX && !kFree) bad = bad || s_lo > 0;
   // Workgroup-wide decision through the last ring stage, which the second
   // walk refills only after its first barrier (the flags are read by then).
   int* const flags = reinterpret_cast<int*>(smem + (NST - 1) * GM::STAGE);
@@ -1258,16 +1396,14 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
     row_sums();
   }
 
-  if constexpr (SEG) {
-    // ---- a segment: unnormalised partials for merge_split_kernel ----
+  if (FLEX && partial >= 0) {
+    // ---- part of a tile: unnormalised partial for the merge ----
     // The partial is (O, l) * 2^m in the scale of exp2(logit): m = 0 for the
     // reference-free pass (log2(block_k) after its correction rescale), the
     // row's reference otherwise (a row that saw no key in its first slice
     // walked without one).
-    const int item = (h * a.split_tiles + (t - (a.Nt - a.split_tiles))) * a.nchunk + chunk;
-    const int64_t base = static_cast<int64_t>(item) * a.nseg + seg;
-    float* const wo = a.ws_o + base * RW * D;
-    float* const wml = a.ws_ml + base * RW * 2;
+    float* const wo = a.ws_o + static_cast<int64_t>(partial) * RW * D;
+    float* const wml = a.ws_ml + static_cast<int64_t>(partial) * RW * 2;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       if (!exists[rt]) continue;
@@ -1302,49 +1438,56 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
   }
 }
 
-// Merge of the split tiles' segments: row r of item (h, tile, chunk) is
-// sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M the largest m_s of the
-// segments with l_s > 0, written as the whole-tile kernel writes it (rows
-// past the valid queries as zeros).  One thread per 4 dims of a row.
+// Merge of a tile's partials: row r is sum_s O_s 2^(m_s - M) / sum_s l_s
+// 2^(m_s - M), M the largest m_s of the partials with l_s > 0, written as the
+// whole-tile kernel writes it (rows past the valid queries as zeros).  One
+// thread per 4 dims of a row.
 template <int D>
 struct MergeShape {
   static constexpr int TPR = D / 4;         // threads per row
-  static constexpr int ROWS = 256 / TPR;    // rows per workgroup
+  static constexpr int ROWS = 256 / TPR;    // rows per workgroup and pass
 };
-template <typename T, int D, int RW>
-__global__ __launch_bounds__(256) void merge_split_kernel(AttnArgs a) {
-  constexpr int TPR = MergeShape<D>::TPR, ROWS = MergeShape<D>::ROWS;
-  constexpr int WPI = (RW + ROWS - 1) / ROWS;  // workgroups per item
-  if (threadIdx.x >= TPR * ROWS) return;
-  const int item = blockIdx.x / WPI;
-  const int r = (blockIdx.x % WPI) * ROWS + threadIdx.x / TPR;
-  const int d0 = (threadIdx.x % TPR) * 4;
-  if (r >= RW) return;
-  const int chunk = item % a.nchunk;
-  const int ht = item / a.nchunk;
-  const int h = ht / a.split_tiles;
-  const int t = a.Nt - a.split_tiles + ht % a.split_tiles;
+// `index(s)`: the s-th partial of the tile.  The loads of kMergeAhead partials
+// are in flight together (the loop is bound by their latency: one at a time,
+// 64 tiles of 9 partials took 33 us).
+constexpr int kMergeAhead = 8;
+template <typename T, int D, int RW, typename F>
+__device__ __forceinline__ void merge_row(const AttnArgs& a, int h, int t, int chunk, int r, int d0, int n, F index) {
   const int prow = chunk * RW + r;
-  if (prow >= a.G * a.tq) return;
+  if (r >= RW || prow >= a.G * a.tq) return;
   const int g = prow / a.tq;
   const int pos = t * a.tq + (prow - g * a.tq);
   if (pos >= a.out_rows) return;
-  const int64_t base = static_cast<int64_t>(item) * a.nseg;
-  float mx = neg_inf();
-  for (int s = 0; s < a.nseg; ++s) {
-    const f32x2 ml = *reinterpret_cast<const f32x2*>(a.ws_ml + ((base + s) * RW + r) * 2);
-    if (ml[1] > 0.f) mx = fmaxf(mx, ml[0]);
-  }
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  float l = 0.f;
-  if (pos < a.Lq && mx != neg_inf()) {
-    for (int s = 0; s < a.nseg; ++s) {
-      const f32x2 ml = *reinterpret_cast<const f32x2*>(a.ws_ml + ((base + s) * RW + r) * 2);
-      if (!(ml[1] > 0.f)) continue;
-      const float w = __builtin_amdgcn_exp2f(ml[0] - mx);
-      const f32x4 o = *reinterpret_cast<const f32x4*>(a.ws_o + ((base + s) * RW + r) * D + d0);
-      acc += o * w;
-      l += ml[1] * w;
+  float l = 0.f, mx = neg_inf();
+  if (pos < a.Lq) {
+    for (int s0 = 0; s0 < n; s0 += kMergeAhead) {
+      f32x2 ml[kMergeAhead];
+      f32x4 o[kMergeAhead];
+#pragma unroll
+      for (int j = 0; j < kMergeAhead; ++j) {
+        const int64_t i = index(min(s0 + j, n - 1)) * RW + r;
+        ml[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + i * 2);
+        o[j] = *reinterpret_cast<const f32x4*>(a.ws_o + i * D + d0);
+      }
+      float m = mx;
+#pragma unroll
+      for (int j = 0; j < kMergeAhead; ++j) {
+        if (s0 + j >= n || !(ml[j][1] > 0.f)) ml[j] = f32x2{neg_inf(), 0.f};
+        m = fmaxf(m, ml[j][0]);
+      }
+      if (m == neg_inf()) continue;  // no key so far
+      const float f = __builtin_amdgcn_exp2f(mx - m);  // (0 while mx = -inf)
+      mx = m;
+      l *= f;
+      acc *= f;
+#pragma unroll
+      for (int j = 0; j < kMergeAhead; ++j) {
+        if (ml[j][0] == neg_inf()) continue;
+        const float w = __builtin_amdgcn_exp2f(ml[j][0] - m);
+        l += ml[j][1] * w;
+        acc += o[j] * w;
+      }
     }
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -1355,23 +1498,58 @@ __global__ __launch_bounds__(256) void merge_split_kernel(AttnArgs a) {
   *reinterpret_cast<u32x2*>(orow + d0) = wv;
 }
 
+// The split dense tail: one workgroup per ROWS rows of an item.
+template <typename T, int D, int RW>
+__global__ __launch_bounds__(256) void merge_split_kernel(AttnArgs a) {
+  constexpr int TPR = MergeShape<D>::TPR, ROWS = MergeShape<D>::ROWS;
+  constexpr int WPI = (RW + ROWS - 1) / ROWS;  // workgroups per item
+  if (threadIdx.x >= TPR * ROWS) return;
+  const int item = blockIdx.x / WPI;
+  const int r = (blockIdx.x % WPI) * ROWS + threadIdx.x / TPR;
+  const int ht = item / a.nchunk;
+  const int64_t base = static_cast<int64_t>(item) * a.nseg;
+  merge_row<T, D, RW>(a, ht / a.split_tiles, a.Nt - a.split_tiles + ht % a.split_tiles, item % a.nchunk, r,
+                      (threadIdx.x % TPR) * 4, a.nseg, [&](int s) { return base + s; });
+}
+
+// The balanced walk: `share` workgroups per item, each for a share of the
+// rows; items walked by one workgroup end at once.
+template <typename T, int D, int RW>
+__global__ __launch_bounds__(256) void merge_balanced_kernel(AttnArgs a, int share) {
+  constexpr int TPR = MergeShape<D>::TPR, ROWS = MergeShape<D>::ROWS;
+  const int e = blockIdx.x / share;
+  const BalCut cut = a.cuts[e];
+  if (cut.first == cut.last || threadIdx.x >= TPR * ROWS) return;
+  const int items = a.split_tiles * a.nchunk;
+  const int h = e / items, item = e % items;
+  const int64_t first = static_cast<int64_t>(h) * a.bal_wgs + cut.first;
+  for (int r = (blockIdx.x % share) * ROWS + threadIdx.x / TPR; r < RW; r += share * ROWS)
+    merge_row<T, D, RW>(a, h, a.Nt - 1 - item / a.nchunk, item % a.nchunk, r, (threadIdx.x % TPR) * 4,
+                        cut.last - cut.first + 1, [&](int s) { return first + s; });
+}
+
 template <int WAVES, int DS>
 constexpr int rows_per_wg() { return WAVES / DS * 32; }
 
-// Split calls: the segments' launch, the whole tiles' launch, then the
-// merge, in stream order.
+// The launch of the parts of the last split_tiles tiles, the whole tiles'
+// launch, then the merge, in stream order.  (One launch of both kinds, the
+// whole tiles walked by the FLEX kernel, was up to 12 % slower: its walk
+// keeps more registers live.)
 template <typename T, int D, bool CORR, int WAVES, int NST, int DS = 1>
 int launch_attn(AttnArgs a, hipStream_t stream) {
   constexpr int RW = rows_per_wg<WAVES, DS>();
   a.nchunk = (a.G * a.tq + RW - 1) / RW;
-  const int64_t seg_wgs = static_cast<int64_t>(a.Hkv) * a.split_tiles * a.nchunk * a.nseg;
+  constexpr int WPI = (RW + MergeShape<D>::ROWS - 1) / MergeShape<D>::ROWS;
+  // workgroups of the last split_tiles tiles (segments or balanced walk)
+  const int64_t part_wgs = a.bal_wgs > 0 ? static_cast<int64_t>(a.Hkv) * a.bal_wgs
+                                         : static_cast<int64_t>(a.Hkv) * a.split_tiles * a.nchunk * a.nseg;
   const int64_t wgs = static_cast<int64_t>(a.Hkv) * (a.Nt - a.split_tiles) * a.nchunk;
-  if (wgs > 0x7fffffffLL || seg_wgs > 0x7fffffffLL)
+  if (wgs > 0x7fffffffLL || part_wgs > 0x7fffffffLL)
     return fail(FPV2_ERR_UNSUPPORTED, "sparse_attention: grid too large");
-  if (seg_wgs > 0) {
+  if (part_wgs > 0) {
     hipLaunchKernelGGL((sparse_attn_kernel<T, D, CORR, WAVES, NST, DS, true>),
-                       dim3(static_cast<unsigned>(seg_wgs)), dim3(WAVES * 64), 0, stream, a);
-    const int rc = check_launch("sparse_attention (segments)");
+                       dim3(static_cast<unsigned>(part_wgs)), dim3(WAVES * 64), 0, stream, a);
+    const int rc = check_launch("sparse_attention (parts)");
     if (rc) return rc;
   }
   if (wgs > 0) {
@@ -1380,11 +1558,18 @@ int launch_attn(AttnArgs a, hipStream_t stream) {
     const int rc = check_launch("sparse_attention");
     if (rc) return rc;
   }
-  if (seg_wgs == 0) return 0;
-  constexpr int WPI = (RW + MergeShape<D>::ROWS - 1) / MergeShape<D>::ROWS;
-  const int64_t mwgs = static_cast<int64_t>(a.Hkv) * a.split_tiles * a.nchunk * WPI;
-  hipLaunchKernelGGL((merge_split_kernel<T, D, RW>), dim3(static_cast<unsigned>(mwgs)), dim3(256), 0,
-                     stream, a);
+  if (part_wgs == 0) return 0;
+  const int64_t items = static_cast<int64_t>(a.Hkv) * a.split_tiles * a.nchunk;
+  if (a.bal_wgs > 0) {
+    // one pass over the rows per workgroup while that stays below 2048
+    // workgroups (most end at once where few items are cut)
+    const int share = static_cast<int>(std::min<int64_t>(WPI, std::max<int64_t>(1, 2048 / items)));
+    hipLaunchKernelGGL((merge_balanced_kernel<T, D, RW>), dim3(static_cast<unsigned>(items * share)), dim3(256), 0,
+                       stream, a, share);
+  } else {
+    hipLaunchKernelGGL((merge_split_kernel<T, D, RW>), dim3(static_cast<unsigned>(items * WPI)), dim3(256), 0,
+                       stream, a);
+  }
   return check_launch("sparse_attention (merge)");
 }
 
@@ -1607,6 +1792,92 @@ extern "C" int fpv2_sparse_attention_split(const void* q, const void* k, const v
     const int64_t items = p->kv_heads * split_tiles * ((G * p->tile_q + kSplitRows - 1) / kSplitRows);
     a.ws_o = static_cast<float*>(workspace);
     a.ws_ml = a.ws_o + items * nseg * kSplitRows * p->head_dim;
+  }
+  return dispatch(a, dtype, p, stream);
+}
+
+// ---------------------------------------------------------------------------
+// Balanced walk of the last `tiles` query tiles.
+// ---------------------------------------------------------------------------
+namespace fpv2 {
+namespace {
+
+// workgroups the chip holds at once: two per compute unit up to D = 128 (256
+// registers a lane), one at D = 256, whose LDS fills it
+int64_t workgroup_slots(const fpv2_attn_params* p) {
+  return static_cast<int64_t>(cu_count()) * (p->head_dim <= 128 ? 2 : 1);
+}
+int64_t balanced_items(const fpv2_attn_params* p, int64_t tiles) {  // (tile, row chunk) items per KV head
+  return tiles * ((p->query_heads / p->kv_heads * p->tile_q + kSplitRows - 1) / kSplitRows);
+}
+// workgroups per KV head: the chip's, and at least one per item
+int64_t balanced_wgs(const fpv2_attn_params* p, int64_t tiles) {
+  return std::max(workgroup_slots(p) / p->kv_heads, balanced_items(p, tiles));
+}
+int64_t balanced_bytes(const fpv2_attn_params* p, int64_t tiles) {
+  return p->kv_heads * (balanced_wgs(p, tiles) * kSplitRows * (p->head_dim + 2) * 4 +
+                        balanced_items(p, tiles) * static_cast<int64_t>(sizeof(BalCut)));
+}
+// Whether the parameters are complete and the sums over a head's items and
+// the grid fit 32 bits.
+bool balanced_ok(const fpv2_attn_params* p, int64_t tiles) {
+  if (!p || p->tile_q <= 0 || p->padded_query_length <= 0 || p->kv_heads <= 0 || p->query_heads <= 0 ||
+      p->query_heads % p->kv_heads || p->block_k <= 0 || p->num_blocks <= 0 || p->head_dim <= 0)
+    return false;
+  if (tiles < 0 || tiles > p->padded_query_length / p->tile_q) return false;
+  const int64_t steps = p->num_blocks * ((p->block_k + 31) / 32 + 1) + 1;
+  return steps < (1LL << 31) && balanced_items(p, tiles) <= ((1LL << 31) - 1) / steps &&
+         p->kv_heads <= 65535 && balanced_wgs(p, tiles) * p->kv_heads <= 0x7fffffffLL / 16;
+}
+
+}  // namespace
+}  // namespace fpv2
+
+extern "C" int64_t fpv2_sparse_attention_balanced_tiles(const fpv2_attn_params* p) {
+  using namespace fpv2;
+  if (!p || p->tile_q <= 0 || !balanced_ok(p, p->padded_query_length / p->tile_q)) return 0;
+  const int64_t tiles = p->padded_query_length / p->tile_q;
+  // Up to half a turn of the chip every item can have two parts.  Measured at
+  // half a turn (D = 128, whole / parts): 499 steps a tile 338 / 238 us, 115
+  // steps 91 / 78 us, 96 steps 75 / 72 us, but 56 steps 48 / 52 us (the merge
+  // launch and the plan); at 0.6 turns 499 steps 358 / 369 us.
+  return balanced_items(p, tiles) * p->kv_heads * 2 <= workgroup_slots(p) ? tiles : 0;
+}
+
+extern "C" int64_t fpv2_sparse_attention_balanced_workspace_bytes(const fpv2_attn_params* p, int64_t tiles) {
+  using namespace fpv2;
+  if (!balanced_ok(p, tiles)) return fail(FPV2_ERR_ARGUMENT, "sparse_attention_balanced: invalid parameters");
+  return tiles == 0 ? 0 : balanced_bytes(p, tiles);
+}
+
+extern "C" int fpv2_sparse_attention_balanced(const void* q, const void* k, const void* v,
+                                              const void* pooled_k, const void* pooled_v,
+                                              const int32_t* selected_ids,
+                                              const int32_t* selected_counts,
+                                              const int32_t* pruned_ids,
+                                              const int32_t* pruned_counts, void* out, int dtype,
+                                              const fpv2_attn_params* p, int64_t tiles,
+                                              void* workspace, int64_t workspace_bytes,
+                                              void* stream) {
+  using namespace fpv2;
+  AttnArgs a{};
+  const int rc = attn_args(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts, pruned_ids,
+                           pruned_counts, out, dtype, p, &a);
+  if (rc) return rc;
+  const int64_t need = fpv2_sparse_attention_balanced_workspace_bytes(p, tiles);
+  if (need < 0) return static_cast<int>(need);
+  if (need > 0) {
+    if (!workspace || workspace_bytes < need)
+      return fail(FPV2_ERR_ARGUMENT, "sparse_attention_balanced: workspace of %lld bytes needed",
+                  static_cast<long long>(need));
+    if (reinterpret_cast<uintptr_t>(workspace) % 16)
+      return fail(FPV2_ERR_ARGUMENT, "sparse_attention_balanced: workspace must be 16-byte aligned");
+    const int64_t wgs = balanced_wgs(p, tiles);
+    a.split_tiles = static_cast<int>(tiles);
+    a.bal_wgs = static_cast<int>(wgs);
+    a.ws_o = static_cast<float*>(workspace);
+    a.ws_ml = a.ws_o + p->kv_heads * wgs * kSplitRows * p->head_dim;
+    a.cuts = reinterpret_cast<BalCut*>(a.ws_ml + p->kv_heads * wgs * kSplitRows * 2);
   }
   return dispatch(a, dtype, p, stream);
 }

@@ -16,6 +16,7 @@ namespace fpv2 {
 void set_error(const char* fmt, ...);
 int fail(int status, const char* fmt, ...);
 int check_launch(const char* kernel);
+int cu_count();  // compute units of the current device
 
 // ---------------------------------------------------------------------------
 // Vector types.  16-bit element types are carried as raw uint16 bits in

@@ -41,6 +41,9 @@ EXPORTED_SYMBOLS = (
     "fpv2_sparse_attention_split_workspace_bytes",
     "fpv2_sparse_attention_split",
     "fpv2_sparse_attention_split_static",
+    "fpv2_sparse_attention_balanced_tiles",
+    "fpv2_sparse_attention_balanced_workspace_bytes",
+    "fpv2_sparse_attention_balanced",
     # decoder-layer operations of the end-to-end harness (fpv2_decoder.h)
     "fpv2_add_rms_norm",
     "fpv2_qk_norm_rope",
@@ -135,6 +138,13 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fpv2_sparse_attention_split_static.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
                                                        i32, ctypes.POINTER(AttnParams), i64, i64,
                                                        vp]
+    lib.fpv2_sparse_attention_balanced_workspace_bytes.restype = i64
+    lib.fpv2_sparse_attention_balanced_workspace_bytes.argtypes = [ctypes.POINTER(AttnParams), i64]
+    lib.fpv2_sparse_attention_balanced_tiles.restype = i64
+    lib.fpv2_sparse_attention_balanced_tiles.argtypes = [ctypes.POINTER(AttnParams)]
+    lib.fpv2_sparse_attention_balanced.restype = ctypes.c_int
+    lib.fpv2_sparse_attention_balanced.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i32,
+                                                   ctypes.POINTER(AttnParams), i64, vp, i64, vp]
     f32 = ctypes.c_float
     lib.fpv2_add_rms_norm.restype = ctypes.c_int
     lib.fpv2_add_rms_norm.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i64, i64, f32, vp]

@@ -267,7 +267,7 @@ class ChunkedPrefill:
             q3, k3, v3, pooled_k, pooled_v, ids, counts, ids, pruned_counts, out,
             device=device, scale=scale, config=config, offset=geo.offset,
             query_length=geo.query_length, key_length=geo.key_length, num_blocks=nb,
-            padded_query_length=geo.padded_query_length, out_rows=geo.query_length)
+            padded_query_length=geo.padded_query_length, out_rows=geo.query_length, balanced=True)
         if marks is not None:
             marks("done")
         if keep is not None:

@@ -232,7 +232,7 @@ def sparse_attention(
         selected_counts, pruned_ids, pruned_counts, out, device=device, scale=scale,
         config=config, offset=offset, query_length=valid_query_length,
         key_length=valid_key_length, num_blocks=num_blocks,
-        padded_query_length=padded_query_length, out_rows=padded_query_length)
+        padded_query_length=padded_query_length, out_rows=padded_query_length, balanced=True)
     return out
 
 
@@ -257,7 +257,8 @@ SPLIT_SEG_STEPS = 128
 def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts,
                       pruned_ids, pruned_counts, out, *, device, scale, config, offset,
                       query_length, key_length, num_blocks, padded_query_length,
-                      out_rows, split_tiles=0, seg_steps=SPLIT_SEG_STEPS) -> None:
+                      out_rows, split_tiles=0, seg_steps=SPLIT_SEG_STEPS,
+                      balanced=False) -> None:
     """Enqueue ``fpv2_sparse_attention`` on the current stream.
 
     ``q``/``k``/``v``/``out`` are ``[H, L, D]`` views (any head and row
@@ -265,7 +266,10 @@ def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts
     are never read.  ``split_tiles``: run the last ``split_tiles`` query
     tiles as key-range segments of ``seg_steps`` sub-tiles, merged after the
     kernel (``fpv2_sparse_attention_split``), with a workspace from the
-    caching allocator.
+    caching allocator.  ``balanced``: cut the walks into parts by their
+    lengths instead, those of the last ``split_tiles`` tiles, or of all tiles
+    where the call has too few to fill the chip
+    (``fpv2_sparse_attention_balanced``).
     """
     lib = _lib.load()
     q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
@@ -284,7 +288,19 @@ def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts
         o_head_stride=out.stride(0), o_row_stride=out.stride(1),
         pooled_head_stride=pooled_k.stride(0))
     with torch.cuda.device(device):
-        if split_tiles:
+        if balanced:
+            split_tiles = lib.fpv2_sparse_attention_balanced_tiles(params) or split_tiles
+        if balanced and split_tiles:
+            need = lib.fpv2_sparse_attention_balanced_workspace_bytes(params, split_tiles)
+            if need < 0:
+                _lib.check(int(need), "sparse_attention_balanced")
+            workspace = torch.empty(int(need), dtype=torch.uint8, device=device)
+            status = lib.fpv2_sparse_attention_balanced(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), pooled_k.data_ptr(),
+                pooled_v.data_ptr(), ids.data_ptr(), counts.data_ptr(), pids.data_ptr(),
+                pcounts.data_ptr(), out.data_ptr(), _lib.dtype_code(q.dtype), params,
+                split_tiles, workspace.data_ptr(), int(need), _lib.stream_ptr(device))
+        elif split_tiles:
             need = lib.fpv2_sparse_attention_split_workspace_bytes(params, split_tiles,
                                                                    seg_steps)
             if need < 0:

@@ -299,8 +299,9 @@ def _select_attend(q3, k3, v3, pooled_k, pooled_v, geo: _Geometry, *, scale, out
     ``out`` (``[Hq, Lq, D]``, allocated when None) and returns it.
     ``hook_stats``: count the call in the hook's ``block_sparsity`` while
     statistics are on (``patch.py:150-155``); callers with counters of
-    their own pass False.  ``split``: tiles to split by key range (None: the
-    dense tail when it is long, ``_dense_tail_split``)."""
+    their own pass False.  ``split``: tiles to split by key range (None: a
+    call of few tiles has them all cut into parts; otherwise the dense tail
+    when it is long, ``_dense_tail_split``)."""
     config = geo.config
     device = q3.device
     lib = _lib.load()
@@ -342,7 +343,7 @@ def _select_attend(q3, k3, v3, pooled_k, pooled_v, geo: _Geometry, *, scale, out
         device=device, scale=scale, config=config, offset=geo.offset,
         query_length=geo.query_length, key_length=geo.key_length, num_blocks=num_blocks,
         padded_query_length=geo.padded_query_length, out_rows=geo.query_length,
-        split_tiles=split_tiles)
+        split_tiles=split_tiles, balanced=split is None)
     if marks is not None:
         marks("done")
     if keep is not None:

@@ -217,6 +217,41 @@ int fpv2_sparse_attention_split(const void* q, const void* k, const void* v,
                                 int64_t seg_steps, void* workspace,
                                 int64_t workspace_bytes, void* stream);
 
+/*
+ * Query tiles of a call whose walks are worth cutting into parts on the
+ * current device (fpv2_sparse_attention_balanced): all of them where whole
+ * tiles would leave half of the chip idle, otherwise 0.
+ */
+int64_t fpv2_sparse_attention_balanced_tiles(const fpv2_attn_params* params);
+
+/*
+ * Workspace bytes of fpv2_sparse_attention_balanced on the current device (0
+ * when tiles is 0), or a negative fpv2_status.
+ */
+int64_t fpv2_sparse_attention_balanced_workspace_bytes(const fpv2_attn_params* params, int64_t tiles);
+
+/*
+ * fpv2_sparse_attention with the walks of the last `tiles` query tiles cut
+ * into parts of similar length, as many as the chip holds workgroups; a
+ * second kernel adds a tile's partials.  For calls with few tiles (a short
+ * chunk of queries, few KV heads, one GPU's share of a layer) and for a dense
+ * tail among sparse tiles.  The parts follow from the list counts, on the
+ * device.  The result equals fpv2_sparse_attention's up to
+ * float32 summation order, the other tiles' rows bit for bit; it is
+ * deterministic.  workspace: at least the bytes above, 16-byte aligned, owned
+ * by the caller (no contents are kept between calls); calls that share a
+ * workspace on different streams race.  No counterpart in the reference
+ * (fpv2/kernel.py:248-325: one threadgroup per query tile).
+ */
+int fpv2_sparse_attention_balanced(const void* q, const void* k, const void* v,
+                                   const void* pooled_k, const void* pooled_v,
+                                   const int32_t* selected_ids,
+                                   const int32_t* selected_counts,
+                                   const int32_t* pruned_ids,
+                                   const int32_t* pruned_counts, void* out, int dtype,
+                                   const fpv2_attn_params* params, int64_t tiles,
+                                   void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Size of the device scratch array of fpv2_sparse_attention_split_static. */
 #define FPV2_SPLIT_SCRATCH_BYTES (64LL << 20)
 

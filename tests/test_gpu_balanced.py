@@ -1,0 +1,170 @@
+"""The balanced walk (``fpv2_sparse_attention_balanced``).
+
+Calls with few query tiles cut the tiles' walks into parts, one workgroup each,
+and add the partials of a tile.  On the same inputs and lists the result must equal the whole-tile
+kernel's up to float32 summation order: both round the same float32 values
+(equal to about 1e-6) to the output type once, so they differ by at most one
+unit in the last place, 2^-7 (bfloat16) or 2^-10 (float16) of the value.
+Where a part of a row takes the online reference, its P words round against
+another reference: half a unit of P per term, 2^-8 of the largest |v| times
+the row's weights, which sum to one (1e-2 below covers |v| < 2.5 averages).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fpv2 import FPV2Config, _lib, pool_blocks
+from fpv2.kernel import _launch_attention, compact_block_indices
+from fpv2.selection import block_scores_and_select
+from fpv2.synthetic import baseline_qkv, structured_qkv
+
+pytestmark = pytest.mark.gpu
+
+ULP = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+
+
+def _lists(q, k, config, pk, n, lk):
+    off = lk - n
+    sel, _ = block_scores_and_select(q, pk, scale=q.shape[-1] ** -0.5, config=config, offset=off,
+                                     query_length=n)
+    return compact_block_indices(sel, config=config, offset=off, query_length=n, key_length=lk)
+
+
+def _both(q, k, v, pk, pv, lists, config, n, lk):
+    outs = []
+    for balanced in (False, True):
+        out = torch.full_like(q, float("nan"))
+        # (all tiles: whether the call would take the walk by itself depends
+        # on its size)
+        _launch_attention(q, k, v, pk, pv, *lists, out, device=q.device,
+                          scale=q.shape[-1] ** -0.5, config=config, offset=lk - n, query_length=n,
+                          key_length=lk, num_blocks=pk.shape[1], padded_query_length=q.shape[1],
+                          out_rows=q.shape[1], balanced=balanced,
+                          split_tiles=q.shape[1] // config.tile_q if balanced else 0)
+        outs.append(out)
+    torch.cuda.synchronize()
+    return outs
+
+
+def _close(whole, even, loose=0.0):
+    assert bool(torch.isfinite(even).all())
+    w, e = whole.float(), even.float()
+    bound = ULP[whole.dtype] * torch.maximum(w.abs(), e.abs()) + 1e-5 + loose
+    assert bool(((w - e).abs() <= bound).all()), float(((w - e).abs() - bound).max())
+
+
+def _pad(x, multiple):
+    n = -(-x.shape[1] // multiple) * multiple
+    out = x.new_zeros((x.shape[0], n, x.shape[2]))
+    out[:, :x.shape[1]] = x
+    return out
+
+
+# (queries, keys): one row; one tile; a last tile of one row; a short chunk of
+# a long prefix; a whole prompt; more items than workgroups of a head
+@pytest.mark.parametrize(("n", "lk"), [(1, 5000), (32, 4096), (65, 3001), (300, 16000),
+                                       (2048, 2048), (2100, 9000)])
+@pytest.mark.parametrize(("d", "dtype", "heads", "corr"), [
+    (128, torch.bfloat16, (4, 1), True), (128, torch.bfloat16, (32, 8), False),
+    (128, torch.float16, (8, 2), True), (64, torch.float16, (16, 2), False),
+    (96, torch.bfloat16, (6, 3), True), (256, torch.bfloat16, (4, 1), True),
+    (256, torch.float16, (4, 4), True),
+])
+def test_equals_whole_tiles(cuda, n, lk, d, dtype, heads, corr):
+    hq, hkv = heads
+    tq = 128 // (hq // hkv)
+    q, k, v = baseline_qkv(lk, query_heads=hq, kv_heads=hkv, head_dim=d, seed=n + d, dtype=dtype,
+                           planted=3.0 * d ** 0.5, heavy_fraction=0.1, device=cuda)
+    q = _pad(q[:, lk - n:], tq)
+    blocks = -(-(lk - n + q.shape[1]) // 128)
+    k, v = (_pad(x, 128 * blocks) for x in (k, v))
+    config = FPV2Config(alpha=0.1, sink_tokens=128, tile_q=tq, mean_correction=corr)
+    pk, pv = pool_blocks(k), pool_blocks(v)
+    lists = _lists(q, k, config, pk, n, lk)
+    whole, even = _both(q, k, v, pk, pv, lists, config, n, lk)
+    # float16 parts after a tile's first walk with the online reference
+    _close(whole, even, 2e-3 if dtype == torch.float16 else 0.0)
+
+
+def test_only_the_last_tiles(cuda):
+    """The dense tail of a long sparse call: the other tiles bit for bit."""
+    n = 8192
+    q, k, v = baseline_qkv(n, planted=3.0 * 128 ** 0.5, seed=7, device=cuda)
+    config = FPV2Config(alpha=0.1, sink_tokens=128, tile_q=32)
+    pk, pv = pool_blocks(k), pool_blocks(v)
+    lists = _lists(q, k, config, pk, n, n)
+    outs = []
+    for tiles in (0, 2):
+        out = torch.empty_like(q)
+        _launch_attention(q, k, v, pk, pv, *lists, out, device=q.device, scale=128 ** -0.5,
+                          config=config, offset=0, query_length=n, key_length=n, num_blocks=64,
+                          padded_query_length=n, out_rows=n, balanced=tiles > 0, split_tiles=tiles)
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0][:, :-64], outs[1][:, :-64])
+    _close(*outs)
+
+
+def test_tiles_of_several_row_chunks_and_a_dense_tail(cuda):
+    """tile_q 128 at G = 4: four 128-row chunks per tile; the last tile is dense."""
+    q, k, v = structured_qkv(length=3072, query_heads=4, kv_heads=1, head_dim=128, seed=5,
+                             dtype=torch.bfloat16, device=cuda)
+    config = FPV2Config(alpha=0.3, sink_tokens=128, window_tokens=128, last_n_blocks=1)
+    pk, pv = pool_blocks(k), pool_blocks(v)
+    lists = _lists(q, k, config, pk, 3072, 3072)
+    assert int(lists[1].max()) > 2 * int(lists[1][:, -2].max())
+    _close(*_both(q, k, v, pk, pv, lists, config, 3072, 3072))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_lists_without_blocks_and_parts_that_overflow(cuda, dtype):
+    """Tiles with empty lists come back as zeros; a key far above the rest in
+    the middle of the walk sends its part to the online walk."""
+    g = torch.Generator().manual_seed(31)
+    n, d = 2048, 128
+    q, k, v = (torch.randn((h, n, d), generator=g) for h in (4, 1, 1))
+    u = torch.randn(d, generator=g)
+    u /= u.norm()
+    k[:, 1000] = 40.0 * u
+    q[:, 1000:] += 40.0 * u
+    q, k, v = (x.to(dtype).to(cuda) for x in (q, k, v))
+    config = FPV2Config(alpha=0.0, sink_tokens=0, window_tokens=0, last_n_blocks=0, tile_q=32,
+                        mean_correction=False)
+    pk, pv = pool_blocks(k), pool_blocks(v)
+    ids, counts, pids, pcounts = _lists(q, k, config, pk, n, n)
+    counts[:, 10:14] = 0
+    whole, even = _both(q, k, v, pk, pv, (ids, counts, pids, pcounts), config, n, n)
+    assert not bool(even[:, 320:448].any())
+    _close(whole, even, 1e-2)
+
+
+def test_workspace_is_checked(cuda):
+    """No tiles where whole tiles fill the chip; a short workspace is refused."""
+    lib = _lib.load()
+
+    def params(length, hq, hkv):
+        nb = length // 128
+        return _lib.AttnParams(
+            query_heads=hq, kv_heads=hkv, head_dim=64, padded_query_length=length,
+            query_length=length, out_rows=length, key_length=length, num_blocks=nb, offset=0,
+            block_k=128, tile_q=32, mean_correction=1, scale=0.125, q_head_stride=length * 64,
+            q_row_stride=64, k_head_stride=length * 64, k_row_stride=64, v_head_stride=length * 64,
+            v_row_stride=64, o_head_stride=length * 64, o_row_stride=64, pooled_head_stride=nb * 64)
+
+    assert lib.fpv2_sparse_attention_balanced_tiles(params(65536, 32, 8)) == 0
+    p = params(1024, 4, 1)
+    assert lib.fpv2_sparse_attention_balanced_tiles(p) == 32
+    assert lib.fpv2_sparse_attention_balanced_workspace_bytes(p, 33) == _lib.FPV2_ERR_ARGUMENT
+    need = lib.fpv2_sparse_attention_balanced_workspace_bytes(p, 32)
+    assert need > 0
+    x = torch.zeros((4, 1024, 64), dtype=torch.bfloat16, device=cuda)
+    lists = torch.zeros((32, 8), dtype=torch.int32, device=cuda)
+    ws = torch.empty(need - 16, dtype=torch.uint8, device=cuda)
+    status = lib.fpv2_sparse_attention_balanced(
+        x.data_ptr(), x.data_ptr(), x.data_ptr(), x.data_ptr(), x.data_ptr(), lists.data_ptr(),
+        lists.data_ptr(), lists.data_ptr(), lists.data_ptr(), torch.empty_like(x).data_ptr(),
+        _lib.BF16, p, 32, ws.data_ptr(), need - 16, _lib.stream_ptr(cuda))
+    assert status == _lib.FPV2_ERR_ARGUMENT
+    assert b"workspace" in lib.fpv2_last_error()
