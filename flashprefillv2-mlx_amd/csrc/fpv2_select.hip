@@ -204,210 +204,184 @@ __device__ void finish_tile(const SelectArgs& a, const TileInfo& ti, float* cb, 
 }
 
 // ---------------------------------------------------------------------------
-// Score-output path: bf16 / f16 queries and pooled keys, head_dim D (multiple
-// of 16), taken when the caller asks for the scores or the scale is not
-// positive (the streaming and owner paths below serve the rest).  Each wave owns 32-block
-// chunks of pooled keys in VGPRs and loops over the pass's row groups.
-// LDS: Q pass [128][D+8] (reused for the flag arrays), c_b[Nb], e_b[Nb].
+// Row path: 16-bit or float32 queries and pooled keys, D in {64, 96, 128,
+// 256}, taken when the caller asks for the scores or for the mask alone, when
+// the scale is not positive and for float32 (the streaming and owner paths
+// below serve the rest).  Each wave owns 32-row groups of the tile and
+// multiplies them with every chunk of 32 pooled keys, both read straight into
+// MFMA fragments (the keys of a head stay in L2): S = Q . Kbar^T, a lane
+// holding 16 rows of one block, from which scores are stored 128 contiguous
+// bytes per row.  Row groups rather than chunks are split over the waves so
+// that short prompts, whose blocks make only one or two chunks, keep every
+// wave busy.  The blocks pass in windows of kRowsWin; each wave sums its own
+// (c, e) per block of the window in LDS, and the waves' pairs are merged at its
+// end.  float32 uses v_mfma_f32_32x32x2_f32: the products and sums stay in
+// float32.
+//   Bound by latency (loads of Q, then of each chunk) and, with scores, by
+// their stores.  Measured at D = 128: 8192 tokens, 32 / 8 heads, bfloat16 with
+// scores 33 us (67 us with one wave per chunk; 134 MB, 27 us at the rate of a
+// copy); 5000 tokens, 8 / 2 heads, float32 34 us (4960 us without MFMA, one
+// thread per block); the mask alone at 15000 tokens 68 us (96 us).
+// LDS: per-wave (c, e) of a window (reused for the flag arrays), c_b[Nb],
+// e_b[Nb].
 // ---------------------------------------------------------------------------
+constexpr int kRowsWin = 512;
+constexpr size_t rows_lds_bytes(int64_t Nb) {
+  return static_cast<size_t>(kThreads / 64) * kRowsWin * 8 + static_cast<size_t>(Nb) * 8;
+}
+static_assert(kThreads / 64 * kRowsWin * 8 >= 2 * FPV2_MAX_BLOCKS, "the flag arrays fit the window's");
+
+// One 16-byte fragment of the products: 8 elements (one MFMA), or 4 floats
+// (four MFMAs of two elements each; both operands order the head dimension
+// alike, so the order does not matter).
+template <typename T>
+__device__ __forceinline__ void rows_mma(u32x4 q, u32x4 k, f32x16& acc) {
+  if constexpr (std::is_same<T, float>::value) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(q[j]), __uint_as_float(k[j]), acc, 0, 0, 0);
+  } else {
+    acc = Elem<T>::mfma32(as_vec8<T>(q), as_vec8<T>(k), acc);
+  }
+}
+
 template <typename T, int D>
-__global__ __launch_bounds__(kThreads, (D <= 128 ? 3 : 2)) void select_mfma_kernel(SelectArgs a) {
-  constexpr int LDQ = D + 8;  // padded row: conflict-free 16-byte column reads
-  constexpr int KS = D / 16;  // MFMA k-steps over the head dimension
+__global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 : 2) <= 512 ? 2 : 1)) void select_rows_kernel(SelectArgs a) {
+  constexpr int ES = std::is_same<T, float>::value ? 4 : 2;  // bytes per element
+  constexpr int NF = D * ES / 32;  // fragments per row and lane half
   extern __shared__ __align__(16) unsigned char smem[];
-  uint16_t* qs = reinterpret_cast<uint16_t*>(smem);
-  float* cb = reinterpret_cast<float*>(smem + kRowsPerPass * LDQ * 2);
-  float* eb = cb + a.Nb;
   __shared__ float fred[4];
   __shared__ int ired[8];
-  __shared__ int rpos[kRowsPerPass];  // local query position, -1: no such row
-  __shared__ int rhead[kRowsPerPass]; // g of the packed row
-  __shared__ int rg_lo[kRowsPerPass / 32], rg_hi[kRowsPerPass / 32];  // per 32-row group
-
   const TileInfo ti = tile_info(a);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int hf = lane >> 5;
+  float* const wc = reinterpret_cast<float*>(smem) + wave * 2 * kRowsWin;  // this wave's c, then e
+  float* const we = wc + kRowsWin;
+  float* const cb = reinterpret_cast<float*>(smem) + 4 * 2 * kRowsWin;
+  float* const eb = cb + a.Nb;
   const int64_t R = a.G * a.tq;
   const int64_t n_comp = a.scores ? a.Nb : ti.nfv;
-  const uint16_t* pk = static_cast<const uint16_t*>(a.pk) + ti.h * a.pk_hs;
-  const uint16_t* qbase = static_cast<const uint16_t*>(a.q);
+  const unsigned char* pk = static_cast<const unsigned char*>(a.pk) + ti.h * a.pk_hs * ES;
+  const unsigned char* qh = static_cast<const unsigned char*>(a.q) + ti.h * a.G * a.q_hs * ES;
   const float sc2 = a.scale * kLog2e;
-  const bool fast_ok = a.scores == nullptr && sc2 > 0.f;
+  const int lq = static_cast<int>(a.Lq);
 
-  for (int64_t b = tid; b < n_comp; b += kThreads) {
-    cb[b] = neg_inf();
-    eb[b] = 0.f;
-  }
-
-  for (int64_t rc = 0; rc < R; rc += kRowsPerPass) {
-    __syncthreads();
-    if (tid < kRowsPerPass) {
-      const int64_t pr = rc + tid;
-      int p = -1, gg = 0;
-      if (pr < R) {
-        gg = static_cast<int>(pr / a.tq);
-        p = static_cast<int>(ti.t * a.tq + (pr - gg * a.tq));
-      }
-      rpos[tid] = p;
-      rhead[tid] = gg;
+  for (int64_t win = 0; win < n_comp; win += kRowsWin) {
+    const int win_n = static_cast<int>(n_comp - win < kRowsWin ? n_comp - win : kRowsWin);
+    for (int i = lane; i < win_n; i += 64) {
+      wc[i] = neg_inf();
+      we[i] = 0.f;
     }
-    __syncthreads();
-    // Lowest and highest position of each 32-row group (-1 rows make the
-    // group take the checked path).
-    if (tid < kRowsPerPass / 32) {
-      int lo_p = 0x7fffffff, hi_p = -1;
-      for (int r = 0; r < 32; ++r) {
-        const int p = rpos[tid * 32 + r];
-        lo_p = min(lo_p, p);
-        hi_p = max(hi_p, p);
+    for (int64_t rc = wave * 32; rc < R; rc += kRowsPerPass) {
+      // this lane's query row (zeros past the tile or the valid length)
+      const int64_t pr = rc + l32;
+      const int64_t g = pr / a.tq;
+      const int pos = pr < R ? static_cast<int>(ti.t * a.tq + (pr - g * a.tq)) : -1;
+      u32x4 qf[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) qf[k] = u32x4{0u, 0u, 0u, 0u};
+      if (pos >= 0 && pos < lq) {
+        const unsigned char* src = qh + (g * a.q_hs + static_cast<int64_t>(pos) * a.q_rs) * ES + hf * 16;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) qf[k] = load16(src + k * 32);
       }
-      rg_lo[tid] = lo_p;
-      rg_hi[tid] = hi_p;
-    }
-    // Stage 128 packed rows of Q (zeros past the tile or the valid length).
-    // For D <= 128 each thread issues all its loads before the stores, so the
-    // staging costs one memory round trip instead of one per load (D = 256
-    // keeps one load at a time: its registers hold no more across the pass).
-    constexpr int QN = kRowsPerPass * (D / 8) / kThreads;
-    static_assert(kRowsPerPass * (D / 8) % kThreads == 0, "Q staging splits evenly");
-    constexpr int QB = D <= 128 ? QN : 1;
-#pragma unroll 1
-    for (int i0 = 0; i0 < QN; i0 += QB) {
-      u32x4 qst[QB];
+      // (wave-uniform) lowest position, and whether every row is present and
+      // inside the valid length
+      int lo_pos = pos, hi_pos = pos;
 #pragma unroll
-      for (int i = 0; i < QB; ++i) {
-        const int e = tid + (i0 + i) * kThreads;
-        const int r = e / (D / 8);
-        const int c = e - r * (D / 8);
-        const int64_t pr = rc + r;
-        qst[i] = u32x4{0u, 0u, 0u, 0u};
-        if (pr < R) {
-          const int64_t g = pr / a.tq;
-          const int64_t pos = ti.t * a.tq + (pr - g * a.tq);
-          if (pos < a.Lq) qst[i] = load16(qbase + (ti.h * a.G + g) * a.q_hs + pos * a.q_rs + c * 8);
-        }
+      for (int o = 16; o >= 1; o >>= 1) {
+        lo_pos = min(lo_pos, __shfl_xor(lo_pos, o));
+        hi_pos = max(hi_pos, __shfl_xor(hi_pos, o));
       }
+      lo_pos = __builtin_amdgcn_readfirstlane(lo_pos);
+      const bool full = lo_pos >= 0 && __builtin_amdgcn_readfirstlane(hi_pos) < lq;
+      // Score rows of the group, from the first one's (rows follow each
+      // other upwards: the padded length covers a tile): byte offsets of the
+      // 16 rows the lane's accumulators hold, rows (j/4)*8 + hf*4 + j%4.
+      const int score_row = static_cast<int>(g * a.Lq_pad) + pos;  // of the KV head (host-checked range)
+      const int score_row0 = __builtin_amdgcn_readfirstlane(score_row);
+      const rsrc_t sr = make_rsrc(a.scores + ((ti.h * a.G * a.Lq_pad) + score_row0) * a.Nb, 0x7fffffffu);
+      uint32_t srow[16];
+      if (a.scores) {
+        const uint32_t mine = pos >= 0 ? static_cast<uint32_t>(score_row - score_row0) * static_cast<uint32_t>(a.Nb) * 4u : kOOB;
 #pragma unroll
-      for (int i = 0; i < QB; ++i) {
-        const int e = tid + (i0 + i) * kThreads;
-        const int r = e / (D / 8);
-        store16(qs + r * LDQ + (e - r * (D / 8)) * 8, qst[i]);
+        for (int j = 0; j < 16; ++j) srow[j] = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3)) + l32 * 4;
       }
-    }
-    __syncthreads();
-    const int64_t rows_here = (R - rc) < kRowsPerPass ? (R - rc) : kRowsPerPass;
-    const int nrg = static_cast<int>((rows_here + 31) / 32);
-    // Lowest / highest row position of the pass (wave-uniform).
-    int pass_lo = 0x7fffffff, pass_hi = -1;
-    for (int rg = 0; rg < nrg; ++rg) {
-      pass_lo = min(pass_lo, rg_lo[rg]);
-      pass_hi = max(pass_hi, rg_hi[rg]);
-    }
-    const int lq = static_cast<int>(a.Lq);
-
-    for (int64_t chunk = wave; chunk * 32 < n_comp; chunk += 4) {
-      const int64_t b = chunk * 32 + l32;
-      // Rows see block b (fully visible blocks only) from local position lo.
-      const bool b_scored = b < ti.nfv;
-      int64_t lo64 = b * a.bk - a.offset;
-      const int lo = lo64 < 0 ? 0 : static_cast<int>(lo64 > 0x7fffffff ? 0x7fffffff : lo64);
-      typename Elem<T>::vec8 kf[KS];
-#pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (b < a.Nb) v = load16(pk + b * D + k * 16 + hf * 8);
-        kf[k] = as_vec8<T>(v);
-      }
-      float cmax = neg_inf(), esum = 0.f;
-      // Fast path: every row of the pass sees the lane's block in every lane
-      // (the chunks before the diagonal), no scores requested, positive
-      // scale: no per-row tests.  The next row group's Q fragments are read
-      // from LDS while the current group's energies are summed.
-      const bool all_ok = b_scored && pass_lo >= lo && pass_hi < lq;
-      if (fast_ok && __ballot(!all_ok) == 0ull) {
-        u32x4 qv[2][KS];
-#pragma unroll
-        for (int k = 0; k < KS; ++k) qv[0][k] = load16(qs + l32 * LDQ + k * 16 + hf * 8);
-        for (int rg = 0; rg < nrg; rg += 2) {
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            const int g = rg + half;
-            if (g < nrg) {
-              f32x16 acc = {};
-#pragma unroll
-              for (int k = 0; k < KS; ++k) acc = Elem<T>::mfma32(as_vec8<T>(qv[half][k]), kf[k], acc);
-              if (g + 1 < nrg) {
-#pragma unroll
-                for (int k = 0; k < KS; ++k)
-                  qv[half ^ 1][k] = load16(qs + ((g + 1) * 32 + l32) * LDQ + k * 16 + hf * 8);
-              }
-              float mx = acc[0];
-#pragma unroll
-              for (int j = 1; j < 16; ++j) mx = fmaxf(mx, acc[j]);
-              const float nc = fmaxf(cmax, mx * sc2);
-              float e0 = (cmax == neg_inf()) ? 0.f : esum * exp2_fast(cmax - nc), e1 = 0.f;
-#pragma unroll
-              for (int j = 0; j < 16; j += 2) {
-                e0 += exp2_fast(fmaf(acc[j], sc2, -nc));
-                e1 += exp2_fast(fmaf(acc[j + 1], sc2, -nc));
-              }
-              cmax = nc;
-              esum = e0 + e1;
-            }
-          }
-        }
-      } else {
-      for (int rg = 0; rg < nrg; ++rg) {
+      for (int c0 = 0; c0 < win_n; c0 += 32) {
+        const int64_t b = win + c0 + l32;
         f32x16 acc = {};
+        {
+          u32x4 kf[NF];
 #pragma unroll
-        for (int k = 0; k < KS; ++k) {
-          const u32x4 qv = load16(qs + (rg * 32 + l32) * LDQ + k * 16 + hf * 8);
-          acc = Elem<T>::mfma32(as_vec8<T>(qv), kf[k], acc);
-        }
-        // Lane holds rows rg*32 + (j/4)*8 + hf*4 + j%4 of block b.
-        float s[16];
-        bool ok[16];
-        float lm = neg_inf();
+          for (int k = 0; k < NF; ++k) kf[k] = u32x4{0u, 0u, 0u, 0u};
+          if (b < a.Nb) {
+            const unsigned char* src = pk + b * D * ES + hf * 16;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int r = rg * 32 + (j >> 2) * 8 + hf * 4 + (j & 3);
-          const int pos = rpos[r];
-          if (a.scores && pos >= 0 && b < a.Nb)
-            a.scores[((ti.h * a.G + rhead[r]) * a.Lq_pad + pos) * a.Nb + b] = acc[j] * a.scale;
-          s[j] = acc[j] * sc2;
-          const bool valid = b_scored && pos >= lo && pos < lq;
-          ok[j] = valid;
-          if (valid) lm = fmaxf(lm, s[j]);
+            for (int k = 0; k < NF; ++k) kf[k] = load16(src + k * 32);
+          }
+#pragma unroll
+          for (int k = 0; k < NF; ++k) rows_mma<T>(qf[k], kf[k], acc);
         }
-        if (lm != neg_inf()) {
-          const float nc = fmaxf(cmax, lm);
-          float e = (cmax == neg_inf()) ? 0.f : esum * exp2_fast(cmax - nc);
+        if (a.scores && b < a.Nb) {
+          const uint32_t at = static_cast<uint32_t>(win + c0) * 4u;
 #pragma unroll
           for (int j = 0; j < 16; ++j)
-            if (ok[j]) e += exp2_fast(s[j] - nc);
-          cmax = nc;
-          esum = e;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[j] * a.scale), sr, srow[j], at, 0);
+        }
+        if (win + c0 >= ti.nfv) continue;  // (uniform) no block of the chunk is scored
+        // Rows that see block b (fully visible blocks only): from local
+        // position lo; the others count as -inf.
+        const int64_t lo64 = b * a.bk - a.offset;
+        const int lo = lo64 < 0 ? 0 : static_cast<int>(lo64 > 0x7fffffff ? 0x7fffffff : lo64);
+        const bool scored = b < ti.nfv;
+        float lm = neg_inf();
+        if (full && __ballot(scored && lo_pos < lo) == 0ull) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            acc[j] = scored ? acc[j] * sc2 : neg_inf();
+            lm = fmaxf(lm, acc[j]);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int p = __shfl(pos, (j >> 2) * 8 + hf * 4 + (j & 3));
+            acc[j] = scored && p >= lo && p < lq ? acc[j] * sc2 : neg_inf();
+            lm = fmaxf(lm, acc[j]);
+          }
+        }
+        float e = 0.f;
+        if (lm != neg_inf()) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) e += exp2_fast(acc[j] - lm);
+        }
+        // the other half of the wave holds the other 16 rows of the group
+        const float oc = __shfl_xor(lm, 32);
+        const float oe = __shfl_xor(e, 32);
+        merge_ce(lm, e, oc, oe);
+        if (hf == 0 && c0 + l32 < win_n) {
+          float c = wc[c0 + l32], s = we[c0 + l32];
+          merge_ce(c, s, lm, e);
+          wc[c0 + l32] = c;
+          we[c0 + l32] = s;
         }
       }
-      }  // checked path
-      // Partner lane (hf ^ 1) holds the other 16 rows of each row group.
-      const float oc = __shfl_xor(cmax, 32);
-      const float oe = __shfl_xor(esum, 32);
-      merge_ce(cmax, esum, oc, oe);
-      if (hf == 0 && b < n_comp) {
-        float c = cb[b], e = eb[b];
-        merge_ce(c, e, cmax, esum);
-        cb[b] = c;
-        eb[b] = e;
-      }
     }
+    __syncthreads();
+    const float* all = reinterpret_cast<const float*>(smem);
+    for (int i = tid; i < win_n; i += kThreads) {
+      float c = all[i], e = all[kRowsWin + i];
+#pragma unroll
+      for (int w = 1; w < kThreads / 64; ++w) merge_ce(c, e, all[w * 2 * kRowsWin + i], all[w * 2 * kRowsWin + kRowsWin + i]);
+      cb[win + i] = c;
+      eb[win + i] = e;
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  // The Q staging area is free now: reuse it for the flag arrays.
-  uint8_t* fsel = reinterpret_cast<uint8_t*>(smem);
+  // the window's arrays are free now: the flag arrays
+  uint8_t* fsel = smem;
   uint8_t* fpr = fsel + a.Nb;
   finish_tile(a, ti, cb, eb, fsel, fpr, fred, ired);
 }
@@ -1326,7 +1300,8 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
 }
 
 // ---------------------------------------------------------------------------
-// Generic path (float32 inputs, or head dims without an MFMA instantiation).
+// Generic path (head dims without an MFMA instantiation, strides or addresses
+// off the 16-byte grid).
 // LDS: Q pass [32][D] float, c_b[Nb], e_b[Nb], flags[2*Nb].
 // ---------------------------------------------------------------------------
 template <typename T>
@@ -1457,6 +1432,27 @@ int launch_generic(K kernel, dim3 grid, size_t lds, hipStream_t stream, const Se
 }
 
 template <typename T>
+int dispatch_rows(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a, bool* done) {
+  // score rows of a head and the byte offsets of a 32-row group's rows in 32
+  // bits (the generic kernel serves the rest)
+  const int64_t heads = a.tq >= 32 ? 2 : 32 / a.tq + 2;  // query heads a row group touches
+  if (a.scores && (a.G * a.Lq_pad >= (1LL << 31) ||
+                   (a.G > 1 && a.tq % 32 ? heads * a.Lq_pad : 32) * a.Nb * 4 >= kMaxRsrcBytes)) {
+    *done = false;
+    return 0;
+  }
+  *done = true;
+  const size_t lds = rows_lds_bytes(a.Nb);
+  switch (D) {
+    case 64: return launch_with_lds(select_rows_kernel<T, 64>, grid, lds, stream, a);
+    case 96: return launch_with_lds(select_rows_kernel<T, 96>, grid, lds, stream, a);
+    case 128: return launch_with_lds(select_rows_kernel<T, 128>, grid, lds, stream, a);
+    case 256: return launch_with_lds(select_rows_kernel<T, 256>, grid, lds, stream, a);
+    default: *done = false; return 0;
+  }
+}
+
+template <typename T>
 int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a, bool* done) {
   *done = true;
   // the hook's paths keep key positions and list entries in 32 bits
@@ -1499,14 +1495,7 @@ int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
       default: break;
     }
   }
-  const size_t tail = static_cast<size_t>(a.Nb) * 8;
-  switch (D) {
-    case 64: return launch_with_lds(select_mfma_kernel<T, 64>, grid, 128 * 72 * 2 + tail, stream, a);
-    case 96: return launch_with_lds(select_mfma_kernel<T, 96>, grid, 128 * 104 * 2 + tail, stream, a);
-    case 128: return launch_with_lds(select_mfma_kernel<T, 128>, grid, 128 * 136 * 2 + tail, stream, a);
-    case 256: return launch_with_lds(select_mfma_kernel<T, 256>, grid, 128 * 264 * 2 + tail, stream, a);
-    default: *done = false; return 0;
-  }
+  return dispatch_rows<T>(D, grid, stream, a, done);
 }
 
 }  // namespace
@@ -1571,13 +1560,15 @@ extern "C" int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
   dim3 grid(static_cast<unsigned>(wgs));
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t D = p->head_dim;
-  const bool vec_ok = D % 8 == 0 && a.q_rs % 8 == 0 && a.q_hs % 8 == 0 && a.pk_hs % 8 == 0 &&
+  const int64_t vec = dtype == FPV2_F32 ? 4 : 8;  // elements per 16-byte access
+  const bool vec_ok = D % vec == 0 && a.q_rs % vec == 0 && a.q_hs % vec == 0 && a.pk_hs % vec == 0 &&
                       reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(pooled_k) % 16 == 0;
   bool done = false;
   int rc = 0;
   if (dtype == FPV2_BF16 && vec_ok) rc = dispatch_mfma<bf16_t>(D, grid, s, a, &done);
   else if (dtype == FPV2_F16 && vec_ok) rc = dispatch_mfma<f16_t>(D, grid, s, a, &done);
+  else if (dtype == FPV2_F32 && vec_ok) rc = dispatch_rows<float>(D, grid, s, a, &done);
   if (done) return rc;
   const size_t lds = static_cast<size_t>(kGenericRows) * D * 4 + static_cast<size_t>(a.Nb) * 10;
   switch (dtype) {

@@ -1,0 +1,96 @@
+"""The row path of block scoring and selection (raw scores, masks without
+lists, non-positive scales, float32), at the edges of its tiles: 32-row
+groups that span query heads or end inside one, 32-block chunks, 512-block
+windows, against the float64 oracle.
+
+Scores are float32 sums of D products accumulated in some order: each of the
+D roundings is at most 2^-24 of the partial sum, so |error| <= D 2^-24
+sum_d |q_d k_d| |scale| (and half an ulp for the scale).  Masks must agree
+outside the 1e-4 band around alpha.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import to_np
+from fpv2 import FPV2Config, block_scores_and_select
+from oracle import fpv2_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+BAND = 1e-4
+
+
+def _cfg(c):
+    return orc.OracleConfig(**{f: getattr(c, f) for f in orc.OracleConfig.__dataclass_fields__})
+
+
+def _check(cuda, dtype, d, heads, tq, nb, qlen, offset, block, scale_sign=1.0, seed=0):
+    hq, hkv = heads
+    g = torch.Generator().manual_seed(seed + nb + d)
+    lq_pad = -(-qlen // tq) * tq
+    q = torch.zeros((hq, lq_pad, d), dtype=dtype)
+    q[:, :qlen] = torch.randn((hq, qlen, d), generator=g).to(dtype)
+    pk = (0.7 * torch.randn((hkv, nb, d), generator=g)).to(dtype)
+    scale = scale_sign * d ** -0.5
+    config = FPV2Config(block_k=block, tile_q=tq, alpha=0.2, sink_tokens=block,
+                        window_tokens=2 * block, last_n_blocks=1)
+    sel, scores = block_scores_and_select(q.to(cuda), pk.to(cuda), scale=scale, config=config,
+                                          offset=offset, query_length=qlen)
+    alone, none = block_scores_and_select(
+        q.to(cuda), pk.to(cuda), scale=scale, offset=offset, query_length=qlen,
+        config=FPV2Config(**{**config.__dict__, "score_chunk_tiles": 2}))
+    assert none is None and torch.equal(sel, alone)
+    qn, kn = to_np(q).astype(np.float64), to_np(pk).astype(np.float64)
+    ref, ref_scores, ratio = orc.block_scores_and_select(
+        qn, kn, scale=scale, config=_cfg(config), offset=offset, query_length=qlen,
+        return_ratio=True)
+    near = np.abs(ratio - config.alpha) <= BAND
+    assert not ((to_np(sel) != ref) & ~near).any()
+    mass = np.einsum("hgnd,hbd->hgnb", np.abs(qn).reshape(hkv, hq // hkv, lq_pad, d), np.abs(kn))
+    bound = (d + 2) * 2.0 ** -24 * mass * abs(scale) + 1e-30
+    assert (np.abs(to_np(scores) - ref_scores) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+@pytest.mark.parametrize(("heads", "tq", "nb", "qlen", "offset"), [
+    ((1, 1), 1, 1, 3, 0),        # one row, one block
+    ((6, 2), 24, 33, 500, 28),   # groups across heads, a chunk of one block
+    ((8, 1), 40, 65, 333, 700),  # several groups per wave, ragged last tile
+    ((4, 4), 160, 31, 450, 40),  # five groups of one head
+])
+def test_scores_and_masks_match_oracle(cuda, dtype, d, heads, tq, nb, qlen, offset):
+    _check(cuda, dtype, d, heads, tq, nb, qlen, offset, 16 if nb > 1 else 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nb", [511, 512, 513, 1100])
+def test_windows_of_blocks(cuda, dtype, nb):
+    """Blocks past the first 512-block window, seen and unseen."""
+    _check(cuda, dtype, 64, (4, 2), 32, nb, 90, nb * 4 - 130, 4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("sign", [-1.0, 0.0])
+def test_scales_that_are_not_positive(cuda, dtype, sign):
+    _check(cuda, dtype, 128, (4, 2), 32, 40, 600, 0, 16, scale_sign=sign)
+
+
+def test_infinite_and_nan_queries_leave_other_tiles_alone(cuda):
+    """A NaN or infinite query row decides its own tiles only; its scores
+    carry it."""
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn((2, 128, 64), generator=g)
+    pk = torch.randn((1, 8, 64), generator=g)
+    config = FPV2Config(block_k=16, tile_q=32, alpha=0.2, sink_tokens=16, window_tokens=16)
+    clean, _ = block_scores_and_select(q.to(cuda), pk.to(cuda), scale=0.125, config=config)
+    q[0, 40, 3] = float("nan")
+    q[1, 70, 5] = float("inf")
+    sel, scores = block_scores_and_select(q.to(cuda), pk.to(cuda), scale=0.125, config=config)
+    assert torch.equal(sel[:, [0, 3]], clean[:, [0, 3]])
+    assert bool(scores[0, 0, 40].isnan().all()) and not bool(scores[0, 1, 70].isfinite().any())
+    assert bool(scores[0, 0, 39].isfinite().all())
