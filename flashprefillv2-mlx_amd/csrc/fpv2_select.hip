@@ -221,7 +221,8 @@ __device__ void finish_tile(const SelectArgs& a, const TileInfo& ti, float* cb, 
 // their stores.  Measured at D = 128: 8192 tokens, 32 / 8 heads, bfloat16 with
 // scores 33 us (67 us with one wave per chunk; 134 MB, 27 us at the rate of a
 // copy); 5000 tokens, 8 / 2 heads, float32 34 us (4960 us without MFMA, one
-// thread per block); the mask alone at 15000 tokens 68 us (96 us).
+// thread per block); the mask alone at 15000 tokens 68 us (96 us; the
+// streaming path takes 45 us and serves it where it can).
 // LDS: per-wave (c, e) of a window (reused for the flag arrays), c_b[Nb],
 // e_b[Nb].
 // ---------------------------------------------------------------------------
@@ -821,7 +822,8 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
 }
 
 // ---------------------------------------------------------------------------
-// Streaming path: the hook's path as a persistent kernel.  Each workgroup
+// Streaming path: the hook's path (and masks without lists or scores, 45 us
+// against the row path's 68 us at 15000 tokens) as a persistent kernel.  Each workgroup
 // walks the tiles bid, bid + grid, ... (latest tiles first) in units of
 // StreamGeom::ROWS packed query rows.  A unit's rows are filled into the
 // LDS slot by asynchronous buffer loads (rows padded by one 16-byte
@@ -1267,6 +1269,12 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
     g_i32* ids = (g_i32*)(fa->ids + row * Nb);
     g_i32* pids = (g_i32*)(fa->pids + row * Nb);
     g_u8* selo = fa->sel_out ? (g_u8*)(fa->sel_out + row * Nb) : nullptr;
+    if (!fa->ids) {  // the mask alone
+      for (int base = w0, it = 0; base < w1; base += 64, ++it)
+        if (base + lane < w1) selo[base + lane] = (selbits >> it) & 1u;
+      for (int b = nvis + tid; b < Nb; b += kThreads) selo[b] = 0;
+      continue;
+    }
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (int base = w0, it = 0; base < w1; base += 64, ++it) {
       const int b = base + lane;
@@ -1464,7 +1472,7 @@ int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
   const bool stream_ok = small && a.tq >= 2 && (a.G * a.tq + 256) * a.tq < (1LL << 32) &&
                          q_span * 2 < kMaxRsrcBytes && a.Nb * D * 2 < kMaxRsrcBytes &&
                          a.Lk > a.offset + (a.Nt - 1) * a.tq && a.Hkv * a.Nt < (1LL << 31);
-  if (a.scores == nullptr && a.scale > 0.f && a.ids != nullptr && stream_ok) {
+  if (a.scores == nullptr && a.scale > 0.f && (a.ids != nullptr || a.sel_out != nullptr) && stream_ok) {
     SelectArgs s = a;
     s.tq_magic = static_cast<uint32_t>(((1ull << 32) + static_cast<uint64_t>(a.tq) - 1) / static_cast<uint64_t>(a.tq));
     const int64_t tiles = a.Hkv * a.Nt;
