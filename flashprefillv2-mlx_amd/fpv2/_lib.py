@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "fpv2_last_error",
     "fpv2_pool_blocks",
     "fpv2_pool_kv",
+    "fpv2_append_pool_kv",
     "fpv2_score_select",
     "fpv2_compact_block_indices",
     "fpv2_sparse_attention",
@@ -118,6 +119,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fpv2_pool_blocks.argtypes = [vp, vp, i32, i64, i64, i64, i64, i64, i64, i64, i64, vp]
     lib.fpv2_pool_kv.restype = ctypes.c_int
     lib.fpv2_pool_kv.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i64, i64, i64, i64, i64, vp]
+    lib.fpv2_append_pool_kv.restype = ctypes.c_int
+    lib.fpv2_append_pool_kv.argtypes = [vp] * 6 + [i32] + [i64] * 13 + [vp]
     lib.fpv2_score_select.restype = ctypes.c_int
     lib.fpv2_score_select.argtypes = [vp, vp, i32, ctypes.POINTER(SelectParams), vp, vp,
                                       vp, vp, vp, vp, vp]

@@ -139,16 +139,47 @@ class ChunkedPrefill:
             raise ValueError(f"{name} must have shape [heads, sequence, dim] or [1, heads, sequence, dim]")
         return x
 
-    def append(self, k: torch.Tensor, v: torch.Tensor) -> None:
-        """Append a chunk's keys and values to the cache."""
+    def _rows(self, k: torch.Tensor, v: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         k, v = self._three_d(k, "k"), self._three_d(v, "v")
         if k.shape != v.shape or k.shape[0] != self.kv_heads or k.shape[-1] != self.head_dim:
             raise ValueError("k and v must be [kv_heads, L, head_dim] of the cache's geometry")
         if k.dtype != self.dtype or v.dtype != self.dtype:
             raise ValueError("q, k, and v must share float16 or bfloat16 dtype")
+        return k, v
+
+    def append(self, k: torch.Tensor, v: torch.Tensor) -> None:
+        """Append a chunk's keys and values to the cache."""
+        k, v = self._rows(k, v)
         k_rows, v_rows = self.reserve(k.shape[1])
         k_rows.copy_(k)
         v_rows.copy_(v)
+
+    def _append_pooled(self, k: torch.Tensor, v: torch.Tensor) -> bool:
+        """``append`` and the pooling of the blocks that gained rows in one
+        launch, where the rows can be read as they are (``step`` only: rows
+        appended by a call of their own may still be edited in the cache
+        before ``attend`` pools them).  False: nothing was done."""
+        k, v = self._rows(k, v)
+        n, old, bk = k.shape[1], self.length, self.config.block_k
+        for x in (k, v):
+            if (x.device != self.k.device or x.requires_grad or x.stride(2) != 1
+                    or x.stride(0) % 8 or x.stride(1) % 8 or x.data_ptr() % 16):
+                return False
+        if n == 0 or type(k) is not torch.Tensor or type(v) is not torch.Tensor:
+            return False
+        self.reserve(n)
+        lib, device = _lib.load(), self.k.device
+        with torch.cuda.device(device):
+            status = lib.fpv2_append_pool_kv(
+                k.data_ptr(), v.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
+                self.pooled_k.data_ptr(), self.pooled_v.data_ptr(), _lib.dtype_code(self.dtype),
+                self.kv_heads, n, old, self._complete, self.head_dim, bk, k.stride(0),
+                k.stride(1), v.stride(0), v.stride(1), self.k.stride(0), self.k.stride(1),
+                self.pooled_k.stride(0), _lib.stream_ptr(device))
+        _lib.check(status, "append_pool_kv")
+        self.pooled_rows += self.length - self._complete * bk
+        self._complete = self.length // bk
+        return True
 
     def reserve(self, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Append ``n`` rows without copying: returns the cache's next ``n``
@@ -201,6 +232,10 @@ class ChunkedPrefill:
         ``out``: optional ``[Hq, L, D]`` destination with any head and row
         stride (D contiguous), e.g. a transposed view of an ``[L, Hq * D]``
         buffer; the result is written there and returned as ``out[None]``."""
+        return self._attend(q, scale=scale, marks=marks, keep=keep, out=out, pooled=False)
+
+    def _attend(self, q, *, scale=None, marks=None, keep=None, out=None, pooled):
+        """``attend``; ``pooled``: the cache's blocks are pooled already."""
         q3 = self._three_d(q, "q")
         if q3.shape[0] != self.query_heads or q3.shape[-1] != self.head_dim:
             raise ValueError("q must be [query_heads, L, head_dim] of the cache's geometry")
@@ -216,7 +251,8 @@ class ChunkedPrefill:
         with torch.cuda.device(device):
             if marks is not None:
                 marks("pool")
-            self._pool_new_blocks(device, lib)
+            if not pooled:
+                self._pool_new_blocks(device, lib)
         if q3.stride(-1) != 1:
             q3 = q3.contiguous()
         if out is None:
@@ -276,5 +312,9 @@ class ChunkedPrefill:
 
     def step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, **kwargs) -> torch.Tensor:
         """Append the chunk's K/V, then attend its queries."""
-        self.append(k, v)
-        return self.attend(q, **kwargs)
+        # (with marks, the pooling is a stage of its own)
+        pooled = kwargs.get("marks") is None and self._append_pooled(k, v)
+        if not pooled:
+            self.append(k, v)
+            return self.attend(q, **kwargs)
+        return self._attend(q, pooled=True, **kwargs)

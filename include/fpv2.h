@@ -131,6 +131,25 @@ int fpv2_pool_kv(const void* k, const void* v, void* pooled_k, void* pooled_v,
                  int64_t pooled_head_stride, void* stream);
 
 /*
+ * Append `rows` rows to the K and V of a cache that holds old_rows rows, and
+ * pool every block that gained rows, in one launch: the rows are copied to
+ * rows [old_rows, old_rows + rows) of k_cache / v_cache, and the blocks from
+ * pooled_blocks (complete blocks whose pooled rows stand already) to the last
+ * partial one are pooled into pooled_k / pooled_v.  k and v have their own
+ * head and row strides, the caches share one pair.  bf16 or f16; head_dim (up
+ * to 512) and strides multiples of 8, rows 16-byte aligned, otherwise
+ * FPV2_ERR_UNSUPPORTED.  The reference appends in the model's cache and pools
+ * the whole prefix per call (fpv2/patch.py:137-138).
+ */
+int fpv2_append_pool_kv(const void* k, const void* v, void* k_cache, void* v_cache,
+                        void* pooled_k, void* pooled_v, int dtype, int64_t kv_heads,
+                        int64_t rows, int64_t old_rows, int64_t pooled_blocks,
+                        int64_t head_dim, int64_t block_size, int64_t k_head_stride,
+                        int64_t k_row_stride, int64_t v_head_stride, int64_t v_row_stride,
+                        int64_t cache_head_stride, int64_t cache_row_stride,
+                        int64_t pooled_head_stride, void* stream);
+
+/*
  * Pooled-QK scoring and block selection, one workgroup per
  * (KV head, query tile); replaces block_scores_and_select,
  * fpv2/selection.py:109-201, fused with compact_block_indices,
