@@ -34,6 +34,7 @@ struct SelectArgs {
   int32_t* pids;
   int32_t* pcounts;
   uint32_t tq_magic;  // ceil(2^32 / tq), streaming path
+  float* parts;  // row path in parts: [tile][part][c, e][Nb]
 };
 
 struct TileInfo {
@@ -220,9 +221,13 @@ __device__ void finish_tile(const SelectArgs& a, const TileInfo& ti, float* cb, 
 //   Bound by latency (loads of Q, then of each chunk) and, with scores, by
 // their stores.  Measured at D = 128: 8192 tokens, 32 / 8 heads, bfloat16 with
 // scores 33 us (67 us with one wave per chunk; 134 MB, 27 us at the rate of a
-// copy); 5000 tokens, 8 / 2 heads, float32 34 us (4960 us without MFMA, one
-// thread per block); the mask alone at 15000 tokens 68 us (96 us; the
+// copy); 5000 tokens, 8 / 2 heads, float32 24 us (34 us with whole tiles; 4960 us
+// without MFMA, one thread per block); the mask alone at 15000 tokens 68 us (96 us; the
 // streaming path takes 45 us and serves it where it can).
+//   Where the call has fewer tiles than the chip holds workgroups and the
+// caller gives a workspace, a tile's row groups are dealt to gridDim.y
+// workgroups (rows_parts): each leaves its (c, e) per block in a.parts, and
+// select_merge_kernel merges a tile's pairs and finishes it.
 // LDS: per-wave (c, e) of a window (reused for the flag arrays), c_b[Nb],
 // e_b[Nb].
 // ---------------------------------------------------------------------------
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
       wc[i] = neg_inf();
       we[i] = 0.f;
     }
-    for (int64_t rc = wave * 32; rc < R; rc += kRowsPerPass) {
+    for (int64_t rc = blockIdx.y * kRowsPerPass + wave * 32; rc < R; rc += gridDim.y * kRowsPerPass) {
       // this lane's query row (zeros past the tile or the valid length)
       const int64_t pr = rc + l32;
       const int64_t g = pr / a.tq;
@@ -376,15 +381,61 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
       float c = all[i], e = all[kRowsWin + i];
 #pragma unroll
       for (int w = 1; w < kThreads / 64; ++w) merge_ce(c, e, all[w * 2 * kRowsWin + i], all[w * 2 * kRowsWin + kRowsWin + i]);
-      cb[win + i] = c;
-      eb[win + i] = e;
+      if (a.parts) {
+        float* const out = a.parts + (static_cast<int64_t>(blockIdx.x) * gridDim.y + blockIdx.y) * 2 * a.Nb + win;
+        out[i] = c;
+        out[a.Nb + i] = e;
+      } else {
+        cb[win + i] = c;
+        eb[win + i] = e;
+      }
     }
     __syncthreads();
   }
+  if (a.parts) return;  // select_merge_kernel finishes the tile
   // the window's arrays are free now: the flag arrays
   uint8_t* fsel = smem;
   uint8_t* fpr = fsel + a.Nb;
   finish_tile(a, ti, cb, eb, fsel, fpr, fred, ired);
+}
+
+// Workgroups that share a tile of the row path: as many as have row groups for
+// all four waves, up to the two workgroups a CU holds, where the tiles fill at
+// most half of the CUs.  Measured with scores at D = 128, whole tiles ->
+// parts: 8 tiles of 512 rows 22.1 -> 12.1 us float32 and 11.9 -> 9.2 us
+// bfloat16, 40 tiles of 1024 rows 60.1 -> 26.9 and 29.5 -> 14.6 us, 96 tiles
+// of 512 rows 44.5 -> 33.5 and 23.0 -> 19.3 us.  At 192 tiles two parts lose
+// (45.0 -> 54.2 and 24.1 -> 26.3 us): the rows already keep most CUs busy and
+// the second launch costs about 5 us.
+int rows_parts(int64_t tiles, int64_t R) {
+  if (2 * tiles > cu_count()) return 1;
+  const int64_t fit = 2LL * cu_count() / tiles;
+  const int64_t full = (R + kRowsPerPass - 1) / kRowsPerPass;
+  const int64_t parts = fit < full ? fit : full;
+  return static_cast<int>(parts < 1 ? 1 : parts);
+}
+
+// Merge the parts' (c, e) of a tile and finish it: one workgroup per tile, in
+// the order of select_rows_kernel's.  Bound by latency (one read of the pairs,
+// then finish_tile's reductions): 4.6 us at 80 tiles of 40 blocks.
+// LDS: c_b[Nb], e_b[Nb], the flag arrays.
+__global__ __launch_bounds__(kThreads) void select_merge_kernel(SelectArgs a, int parts) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ float fred[4];
+  __shared__ int ired[8];
+  const TileInfo ti = tile_info(a);
+  float* const cb = reinterpret_cast<float*>(smem);
+  float* const eb = cb + a.Nb;
+  const float* const src = a.parts + static_cast<int64_t>(blockIdx.x) * parts * 2 * a.Nb;
+  for (int64_t b = threadIdx.x; b < ti.nfv; b += kThreads) {
+    float c = neg_inf(), e = 0.f;
+    for (int p = 0; p < parts; ++p) merge_ce(c, e, src[2 * p * a.Nb + b], src[(2 * p + 1) * a.Nb + b]);
+    cb[b] = c;
+    eb[b] = e;
+  }
+  __syncthreads();
+  uint8_t* const fsel = reinterpret_cast<uint8_t*>(eb + a.Nb);
+  finish_tile(a, ti, cb, eb, fsel, fsel + a.Nb, fred, ired);
 }
 
 // ---------------------------------------------------------------------------
@@ -1451,13 +1502,27 @@ int dispatch_rows(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
   }
   *done = true;
   const size_t lds = rows_lds_bytes(a.Nb);
+  SelectArgs s = a;
+  const dim3 tiles = grid;
+  const int parts = a.parts ? rows_parts(tiles.x, a.G * a.tq) : 1;
+  grid.y = static_cast<unsigned>(parts);
+  if (parts == 1) s.parts = nullptr;
+  int rc;
   switch (D) {
-    case 64: return launch_with_lds(select_rows_kernel<T, 64>, grid, lds, stream, a);
-    case 96: return launch_with_lds(select_rows_kernel<T, 96>, grid, lds, stream, a);
-    case 128: return launch_with_lds(select_rows_kernel<T, 128>, grid, lds, stream, a);
-    case 256: return launch_with_lds(select_rows_kernel<T, 256>, grid, lds, stream, a);
+    case 64: rc = launch_with_lds(select_rows_kernel<T, 64>, grid, lds, stream, s); break;
+    case 96: rc = launch_with_lds(select_rows_kernel<T, 96>, grid, lds, stream, s); break;
+    case 128: rc = launch_with_lds(select_rows_kernel<T, 128>, grid, lds, stream, s); break;
+    case 256: rc = launch_with_lds(select_rows_kernel<T, 256>, grid, lds, stream, s); break;
     default: *done = false; return 0;
   }
+  if (rc || parts == 1) return rc;
+  const size_t merge_lds = static_cast<size_t>(a.Nb) * 10;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(select_merge_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          static_cast<int>(merge_lds)) != hipSuccess)
+    return fail(FPV2_ERR_LAUNCH, "score_select: hipFuncSetAttribute failed");
+  hipLaunchKernelGGL(select_merge_kernel, tiles, dim3(kThreads), merge_lds, stream, s, parts);
+  return check_launch("score_select");
 }
 
 template <typename T>
@@ -1506,14 +1571,21 @@ int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
   return dispatch_rows<T>(D, grid, stream, a, done);
 }
 
-}  // namespace
-}  // namespace fpv2
+// Bytes of the row path's workspace (0: a tile stays in one workgroup).  The
+// sizes are checked by score_select; what it refuses needs none.
+int64_t rows_workspace(const fpv2_select_params* p) {
+  if (!p || p->kv_heads <= 0 || p->query_heads <= 0 || p->query_heads % p->kv_heads || p->tile_q <= 0 ||
+      p->padded_query_length <= 0 || p->num_blocks <= 0 || p->num_blocks > FPV2_MAX_BLOCKS)
+    return 0;
+  const int64_t tiles = p->padded_query_length / p->tile_q;
+  if (tiles <= 0 || tiles > cu_count() || p->kv_heads > cu_count() || p->tile_q > (1LL << 31)) return 0;
+  const int parts = rows_parts(p->kv_heads * tiles, p->query_heads / p->kv_heads * p->tile_q);
+  return parts > 1 ? p->kv_heads * tiles * parts * 2 * p->num_blocks * 4 : 0;
+}
 
-extern "C" int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
-                                 const fpv2_select_params* p, uint8_t* selected, float* scores,
-                                 int32_t* selected_ids, int32_t* selected_counts,
-                                 int32_t* pruned_ids, int32_t* pruned_counts, void* stream) {
-  using namespace fpv2;
+int score_select(const void* q, const void* pooled_k, int dtype, const fpv2_select_params* p,
+                 uint8_t* selected, float* scores, int32_t* selected_ids, int32_t* selected_counts,
+                 int32_t* pruned_ids, int32_t* pruned_counts, float* parts, void* stream) {
   if (!p || !q || !pooled_k) return fail(FPV2_ERR_ARGUMENT, "score_select: null argument");
   if (p->kv_heads <= 0 || p->query_heads <= 0 || p->query_heads % p->kv_heads)
     return fail(FPV2_ERR_ARGUMENT, "query heads must be divisible by KV heads");
@@ -1563,6 +1635,7 @@ extern "C" int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
   a.counts = selected_counts;
   a.pids = pruned_ids;
   a.pcounts = pruned_counts;
+  a.parts = parts;
   const int64_t wgs = a.Hkv * a.Nt;
   if (wgs > 0x7fffffffLL) return fail(FPV2_ERR_UNSUPPORTED, "score_select: grid too large");
   dim3 grid(static_cast<unsigned>(wgs));
@@ -1585,6 +1658,36 @@ extern "C" int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
     case FPV2_F16: return launch_generic(select_generic_kernel<f16_t>, grid, lds, s, a, static_cast<int>(D));
     default: return fail(FPV2_ERR_UNSUPPORTED, "score_select: unsupported dtype %d", dtype);
   }
+}
+
+}  // namespace
+}  // namespace fpv2
+
+extern "C" int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
+                                 const fpv2_select_params* p, uint8_t* selected, float* scores,
+                                 int32_t* selected_ids, int32_t* selected_counts,
+                                 int32_t* pruned_ids, int32_t* pruned_counts, void* stream) {
+  return fpv2::score_select(q, pooled_k, dtype, p, selected, scores, selected_ids, selected_counts,
+                            pruned_ids, pruned_counts, nullptr, stream);
+}
+
+extern "C" int64_t fpv2_score_select_workspace_bytes(const fpv2_select_params* p) {
+  return fpv2::rows_workspace(p);
+}
+
+extern "C" int fpv2_score_select_parts(const void* q, const void* pooled_k, int dtype,
+                                       const fpv2_select_params* p, uint8_t* selected, float* scores,
+                                       int32_t* selected_ids, int32_t* selected_counts,
+                                       int32_t* pruned_ids, int32_t* pruned_counts,
+                                       void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace fpv2;
+  const int64_t need = rows_workspace(p);
+  if (need > 0 && (!workspace || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16))
+    return fail(FPV2_ERR_ARGUMENT, "score_select: the workspace must be 16-byte aligned and hold %lld bytes",
+                static_cast<long long>(need));
+  return score_select(q, pooled_k, dtype, p, selected, scores, selected_ids, selected_counts,
+                      pruned_ids, pruned_counts, need > 0 ? static_cast<float*>(workspace) : nullptr,
+                      stream);
 }
 
 extern "C" int fpv2_compact_block_indices(const uint8_t* selected, int64_t kv_heads,

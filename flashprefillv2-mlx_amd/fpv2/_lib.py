@@ -37,6 +37,8 @@ EXPORTED_SYMBOLS = (
     "fpv2_pool_kv",
     "fpv2_append_pool_kv",
     "fpv2_score_select",
+    "fpv2_score_select_parts",
+    "fpv2_score_select_workspace_bytes",
     "fpv2_compact_block_indices",
     "fpv2_sparse_attention",
     "fpv2_sparse_attention_split_workspace_bytes",
@@ -124,6 +126,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fpv2_score_select.restype = ctypes.c_int
     lib.fpv2_score_select.argtypes = [vp, vp, i32, ctypes.POINTER(SelectParams), vp, vp,
                                       vp, vp, vp, vp, vp]
+    lib.fpv2_score_select_workspace_bytes.restype = i64
+    lib.fpv2_score_select_workspace_bytes.argtypes = [ctypes.POINTER(SelectParams)]
+    lib.fpv2_score_select_parts.restype = ctypes.c_int
+    lib.fpv2_score_select_parts.argtypes = [vp, vp, i32, ctypes.POINTER(SelectParams), vp, vp,
+                                            vp, vp, vp, vp, vp, i64, vp]
     lib.fpv2_compact_block_indices.restype = ctypes.c_int
     lib.fpv2_compact_block_indices.argtypes = [vp, i64, i64, i64, i64, i64, i64, i64,
                                                vp, vp, vp, vp, vp]

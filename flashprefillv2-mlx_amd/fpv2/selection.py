@@ -198,10 +198,20 @@ def block_scores_and_select(
                             padded_length=padded_length,
                             key_length=num_blocks * config.block_k)
     with torch.cuda.device(device):
-        status = lib.fpv2_score_select(
-            qk.data_ptr(), pk.data_ptr(), _lib.dtype_code(dtype), params,
-            selected.data_ptr(), _lib.ptr(scores), None, None, None, None,
-            _lib.stream_ptr(device))
+        # (a mask of 16-bit inputs alone takes the streaming path, which has no use for it)
+        rows = scores is not None or dtype == torch.float32 or not scale > 0
+        need = lib.fpv2_score_select_workspace_bytes(params) if rows else 0
+        if need:
+            workspace = torch.empty(int(need), dtype=torch.uint8, device=device)
+            status = lib.fpv2_score_select_parts(
+                qk.data_ptr(), pk.data_ptr(), _lib.dtype_code(dtype), params,
+                selected.data_ptr(), _lib.ptr(scores), None, None, None, None,
+                workspace.data_ptr(), int(need), _lib.stream_ptr(device))
+        else:
+            status = lib.fpv2_score_select(
+                qk.data_ptr(), pk.data_ptr(), _lib.dtype_code(dtype), params,
+                selected.data_ptr(), _lib.ptr(scores), None, None, None, None,
+                _lib.stream_ptr(device))
     _lib.check(status, "block_scores_and_select")
     return selected, scores
 

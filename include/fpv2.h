@@ -169,6 +169,21 @@ int fpv2_score_select(const void* q, const void* pooled_k, int dtype,
                       int32_t* pruned_counts, void* stream);
 
 /*
+ * fpv2_score_select with a workspace (16-byte aligned device memory) of
+ * fpv2_score_select_workspace_bytes bytes for the current device (0: none
+ * needed, workspace may be NULL).  Calls of few tiles that return the scores,
+ * take float32 or a scale that is not positive then share a tile's rows among
+ * several workgroups, whose energies a second launch merges.
+ */
+int64_t fpv2_score_select_workspace_bytes(const fpv2_select_params* params);
+int fpv2_score_select_parts(const void* q, const void* pooled_k, int dtype,
+                            const fpv2_select_params* params, uint8_t* selected,
+                            float* scores, int32_t* selected_ids,
+                            int32_t* selected_counts, int32_t* pruned_ids,
+                            int32_t* pruned_counts, void* workspace,
+                            int64_t workspace_bytes, void* stream);
+
+/*
  * Compact a selection mask into padded ascending block lists:
  * selected_ids = selected blocks ascending, then unselected ascending
  * (a stable argsort of -mask); pruned = ~selected & (min(block_end,
