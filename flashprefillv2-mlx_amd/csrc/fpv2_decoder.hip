@@ -227,6 +227,54 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(SiluArgs a) {
   }
 }
 
+struct LogitsArgs {
+  const uint16_t* x;
+  const uint16_t* w;
+  float* out;
+  int64_t vocab, cols, w_stride;
+};
+
+// One position's logits: out[v] = sum_c x[c] w[v][c] in float32.  Bound by the
+// read of the weights.  A wave takes kLogitRows rows at a time, so that each
+// lane has that many 16-byte loads in flight per 512 columns, and adds the
+// lanes' sums at the end; x stays in L1.  151936 rows
+// of 2560 bfloat16: 137 us, 5.7 TB/s (242 us as a library product of one row).
+constexpr int kLogitRows = 4;
+
+template <typename T>
+__global__ __launch_bounds__(256) void row_logits_kernel(LogitsArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t v0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kLogitRows;
+  if (v0 >= a.vocab) return;
+  const uint16_t* row[kLogitRows];
+  float sum[kLogitRows];
+#pragma unroll
+  for (int r = 0; r < kLogitRows; ++r) {
+    row[r] = a.w + (v0 + r < a.vocab ? v0 + r : a.vocab - 1) * a.w_stride;
+    sum[r] = 0.f;
+  }
+#pragma unroll 5
+  for (int64_t c = lane * 8; c < a.cols; c += 512) {
+    u32x4 wv[kLogitRows];
+#pragma unroll
+    for (int r = 0; r < kLogitRows; ++r) wv[r] = *reinterpret_cast<const u32x4*>(row[r] + c);
+    const u32x4 xv = *reinterpret_cast<const u32x4*>(a.x + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lo = lo_f<T>(xv[j]), hi = hi_f<T>(xv[j]);
+#pragma unroll
+      for (int r = 0; r < kLogitRows; ++r)
+        sum[r] = fmaf(hi, hi_f<T>(wv[r][j]), fmaf(lo, lo_f<T>(wv[r][j]), sum[r]));
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kLogitRows; ++r) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) sum[r] += __shfl_xor(sum[r], o);
+    if (lane == 0 && v0 + r < a.vocab) a.out[v0 + r] = sum[r];
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -338,4 +386,29 @@ extern "C" int fpv2_silu_mul(const void* gate_up, void* out, int dtype, int64_t 
   else
     hipLaunchKernelGGL(silu_mul_kernel<f16_t>, dim3(grid), dim3(256), 0, s, a);
   return check_launch("silu_mul_kernel");
+}
+
+extern "C" int fpv2_row_logits(const void* x, const void* weight, float* out, int dtype,
+                               int64_t vocab, int64_t cols, int64_t weight_row_stride,
+                               void* stream) {
+  using namespace fpv2;
+  if (dtype != FPV2_BF16 && dtype != FPV2_F16)
+    return fail(FPV2_ERR_UNSUPPORTED, "fpv2_row_logits: dtype must be bf16 or f16");
+  if (!x || !weight || !out) return fail(FPV2_ERR_ARGUMENT, "fpv2_row_logits: null pointer");
+  if (vocab < 0 || cols <= 0 || cols % 8 || weight_row_stride < cols || weight_row_stride % 8)
+    return fail(FPV2_ERR_ARGUMENT, "fpv2_row_logits: cols and the row stride must be multiples "
+                "of 8, weight_row_stride >= cols");
+  if (!aligned16(x) || !aligned16(weight))
+    return fail(FPV2_ERR_ARGUMENT, "fpv2_row_logits: pointers must be 16-byte aligned");
+  if (vocab == 0) return FPV2_OK;
+  const int64_t grid = (vocab + 4 * kLogitRows - 1) / (4 * kLogitRows);
+  if (grid > 0x7fffffff) return fail(FPV2_ERR_ARGUMENT, "fpv2_row_logits: too many rows");
+  LogitsArgs a{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight), out, vocab,
+               cols, weight_row_stride};
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == FPV2_BF16)
+    hipLaunchKernelGGL(row_logits_kernel<bf16_t>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(row_logits_kernel<f16_t>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, a);
+  return check_launch("row_logits_kernel");
 }

@@ -51,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "fpv2_add_rms_norm",
     "fpv2_qk_norm_rope",
     "fpv2_silu_mul",
+    "fpv2_row_logits",
 )
 
 
@@ -163,6 +164,8 @@ def _declare(lib: ctypes.CDLL) -> None:
                                       i64, i64, i64, i64, i64, f32, vp]
     lib.fpv2_silu_mul.restype = ctypes.c_int
     lib.fpv2_silu_mul.argtypes = [vp, vp, i32, i64, i64, i64, i64, vp]
+    lib.fpv2_row_logits.restype = ctypes.c_int
+    lib.fpv2_row_logits.argtypes = [vp, vp, vp, i32, i64, i64, i64, vp]
 
 
 def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:

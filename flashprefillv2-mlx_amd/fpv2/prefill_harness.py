@@ -139,6 +139,23 @@ def _silu_mul(gate_up: torch.Tensor, cols: int) -> torch.Tensor:
     return out
 
 
+def _row_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """float32 ``weight @ x`` of one row ``x`` (``fpv2_row_logits``)."""
+    lib = _lib.load()
+    if x.ndim != 1 or weight.shape[1:] != x.shape or x.stride(0) != 1 or weight.stride(1) != 1:
+        raise ValueError("weight must be [vocab, cols] and x [cols], with contiguous columns")
+    if weight.dtype != x.dtype:
+        raise ValueError("x and weight must share a dtype")
+    _lib.require_device(x, weight)
+    out = torch.empty(weight.shape[0], dtype=torch.float32, device=x.device)
+    with torch.cuda.device(x.device):
+        status = lib.fpv2_row_logits(
+            x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(x.dtype),
+            weight.shape[0], weight.shape[1], weight.stride(0), _lib.stream_ptr(x.device))
+    _lib.check(status, "fpv2_row_logits")
+    return out
+
+
 def rope_tables(shape: DecoderShape, positions: torch.Tensor):
     """cos/sin ``[L, D]`` of rotate-half RoPE for integer positions."""
     half = shape.head_dim // 2
@@ -327,7 +344,7 @@ class ChunkedPrefillRunner:
             for li in range(m.shape.layers):
                 x, delta = self._layer(li, x, delta, cos, sin)
         last = _add_rms_norm(x[-1:], delta[-1:], m.final_norm, m.shape.rms_eps)
-        return F.linear(last, m.embed).float()[0]
+        return _row_logits(last[0], m.embed)
 
 
 def measure(shape: DecoderShape, *, tokens: int, chunk: int, alpha: float, device,

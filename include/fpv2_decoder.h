@@ -77,6 +77,16 @@ int fpv2_silu_mul(const void* gate_up, void* out, int dtype, int64_t rows,
                   int64_t cols, int64_t in_row_stride, int64_t out_row_stride,
                   void* stream);
 
+/*
+ * Logits of one position: out[v] = sum_c x[c] weight[v][c], products and sums
+ * in float32.  cols and weight_row_stride multiples of 8, x and weight
+ * 16-byte aligned.
+ * Counterpart of mlx-lm's tied head (embed_tokens.as_linear) on the last row.
+ */
+int fpv2_row_logits(const void* x, const void* weight, float* out, int dtype,
+                    int64_t vocab, int64_t cols, int64_t weight_row_stride,
+                    void* stream);
+
 #ifdef __cplusplus
 }
 #endif
