@@ -1439,7 +1439,7 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
 }
 
 // Merge of a tile's partials: row r is sum_s O_s 2^(m_s - M) / sum_s l_s
-// 2^(m_s - M), M the largest m_s of the partials with l_s > 0, written as the
+// 2^(m_s - M), M the largest m_s of the partials with l_s != 0, written as the
 // whole-tile kernel writes it (rows past the valid queries as zeros).  One
 // thread per 4 dims of a row.
 template <int D>
@@ -1470,21 +1470,28 @@ __device__ __forceinline__ void merge_row(const AttnArgs& a, int h, int t, int c
         ml[j] = *reinterpret_cast<const f32x2*>(a.ws_ml + i * 2);
         o[j] = *reinterpret_cast<const f32x4*>(a.ws_o + i * D + d0);
       }
+      // A partial without a key (l == 0) has O = 0, or NaN from a V row that
+      // no key of its own weights (0 x inf, 0 x NaN), and does not set the
+      // scale.  A NaN l is a key: it passes into the row as it does into a
+      // whole tile's.
       float m = mx;
 #pragma unroll
       for (int j = 0; j < kMergeAhead; ++j) {
-        if (s0 + j >= n || !(ml[j][1] > 0.f)) ml[j] = f32x2{neg_inf(), 0.f};
+        if (s0 + j >= n) {
+          ml[j] = f32x2{neg_inf(), 0.f};
+          o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (ml[j][1] == 0.f) ml[j][0] = neg_inf();
         m = fmaxf(m, ml[j][0]);
       }
-      if (m == neg_inf()) continue;  // no key so far
-      const float f = __builtin_amdgcn_exp2f(mx - m);  // (0 while mx = -inf)
+      // (equal scales, infinite ones too, have the factor 1)
+      const float f = mx == m ? 1.f : __builtin_amdgcn_exp2f(mx - m);
       mx = m;
       l *= f;
       acc *= f;
 #pragma unroll
       for (int j = 0; j < kMergeAhead; ++j) {
-        if (ml[j][0] == neg_inf()) continue;
-        const float w = __builtin_amdgcn_exp2f(ml[j][0] - m);
+        const float w = ml[j][1] == 0.f ? 0.f : (ml[j][0] == m ? 1.f : __builtin_amdgcn_exp2f(ml[j][0] - m));
         l += ml[j][1] * w;
         acc += o[j] * w;
       }

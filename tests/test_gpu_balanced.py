@@ -140,6 +140,52 @@ def test_lists_without_blocks_and_parts_that_overflow(cuda, dtype):
     _close(whole, even, 1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("d", "corr"), [(64, True), (128, False), (256, True)])
+@pytest.mark.parametrize(("where", "value"), [
+    ("q", "nan"), ("q", "inf"), ("k", "nan"), ("k", "inf"), ("v", "nan"),
+    ("v", "inf"), ("rows", "nan")])
+def test_infinities_and_nan_reach_the_rows_they_reach_whole(cuda, dtype, d, corr, where, value):
+    """A NaN or infinite query row, a key row in a middle part, a value row
+    that later rows see and the tile's earlier rows only multiply by zero, and
+    NaN query rows of whole tiles: the output is NaN and infinite exactly where
+    a whole tile's is.  Also through ``out`` of other strides."""
+    g = torch.Generator().manual_seed(d)
+    n, lk = 200, 5000
+    q, k, v = (torch.randn((h, m, d), generator=g) for h, m in ((8, n), (2, lk), (2, lk)))
+    x = float(value)
+    if where == "q":
+        q[3, 70, 2] = x
+    elif where == "rows":
+        q[:, 60:130] = x
+    elif where == "k":
+        k[0, 2100, 1] = x
+    else:
+        v[1, lk - 60, 3] = x
+    q, k, v = (t.to(dtype).to(cuda) for t in (q, k, v))
+    config = FPV2Config(alpha=0.1, sink_tokens=128, tile_q=32, mean_correction=corr)
+    q, blocks = _pad(q, 32), -(-(lk - n + -(-n // 32) * 32) // 128)
+    k, v = (_pad(t, 128 * blocks) for t in (k, v))
+    # (lists of the finite inputs: every tile keeps some and prunes some)
+    mask = torch.ones((2, q.shape[1] // 32, blocks), dtype=torch.bool, device=cuda)
+    mask[:, :, 4:9] = False
+    lists = compact_block_indices(mask, config=config, offset=lk - n, query_length=n, key_length=lk)
+    pk, pv = pool_blocks(k), pool_blocks(v)
+    whole, even = (o[:, :n].float() for o in _both(q, k, v, pk, pv, lists, config, n, lk))
+    assert torch.equal(whole.isnan(), even.isnan()) and torch.equal(whole.isinf(), even.isinf())
+    keep = whole.isfinite()
+    assert not bool(keep.all())
+    _close(whole[keep].to(dtype), even[keep].to(dtype), 1e-2)
+    wide = torch.full((n, 8, d + 8), float("nan"), dtype=dtype, device=cuda)
+    _launch_attention(q, k, v, pk, pv, *lists, wide[:, :, :d].transpose(0, 1), device=q.device,
+                      scale=d ** -0.5, config=config, offset=lk - n, query_length=n, key_length=lk,
+                      num_blocks=blocks, padded_query_length=q.shape[1], out_rows=n, balanced=True,
+                      split_tiles=q.shape[1] // 32)
+    assert torch.equal(wide[:, :, :d].transpose(0, 1).float().nan_to_num(7.0, 8.0, 9.0),
+                       even.nan_to_num(7.0, 8.0, 9.0))
+    assert bool(wide[:, :, d:].isnan().all())
+
+
 def test_workspace_is_checked(cuda):
     """No tiles where whole tiles fill the chip; a short workspace is refused."""
     lib = _lib.load()
