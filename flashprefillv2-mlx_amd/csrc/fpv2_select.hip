@@ -925,7 +925,12 @@ struct StreamGeom {
 // list counts [8]
 constexpr size_t stream_lds_bytes(int64_t Nb) { return static_cast<size_t>(Nb) * 4 + (256 + 4 + 4 + 8) * 4; }
 
-template <typename T, int D, bool SWZ>
+// MASK: the mask alone, for block_scores_and_select, whose masks of inputs with
+// infinities and NaN must be the row path's, which serves the same call with
+// scores: of the 16 rows a lane holds at a time, those without a logit above
+// -inf add nothing, and otherwise a NaN or +inf logit makes the block's energy
+// NaN.  (The hook's lists take a sum that is NaN as it comes.)
+template <typename T, int D, bool SWZ, bool MASK>
 __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) void select_stream_kernel(
     SelectArgs a) {
   using SG = StreamGeom<D, SWZ>;
@@ -1155,8 +1160,10 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
         float lm = neg_inf();
 #pragma unroll
         for (int j = 0; j < 16; ++j) lm = ok(j) ? fmaxf(lm, s[j]) : lm;
-        const float m_new = wave_max_dpp(lm) * sc2;
-        const float f = (mref == neg_inf()) ? 0.f : exp2_fast(mref - m_new);
+        const float top = wave_max_dpp(lm) * sc2;
+        // (MASK: also entered for a NaN sum, whose wave may need no raise)
+        const float m_new = MASK ? fmaxf(mref, top) : top;
+        const float f = (mref == neg_inf()) ? 0.f : (MASK && mref == m_new) ? 1.f : exp2_fast(mref - m_new);
         eacc *= f;
         emax_w *= f;
         for (int cc = wave; cc < nchunks; cc += 4) {
@@ -1164,7 +1171,11 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
           if (hf == 0 && bb < nfv) eb[bb] *= f;
         }
         mref = m_new;
+        const float e = exp_sum(s, ok);
+        return MASK && lm == neg_inf() ? 0.f : e;
       };
+      // whether the sum needs another reference (MASK: or is NaN)
+      auto off = [](float e) { return __ballot(MASK ? !(e <= kRaiseSum) : e > kRaiseSum) != 0ull; };
       // add the chunk's energies (both halves of the wave) to E_b
       auto store_chunk = [&](int b, bool b_scored, float eacc) {
         const auto es = __builtin_amdgcn_permlane32_swap(__float_as_uint(eacc), __float_as_uint(eacc), false, false);
@@ -1210,10 +1221,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
                 __builtin_amdgcn_sched_group_barrier(0x002, 48 / KS, 0);
               }
             }
-            if (__ballot(e > kRaiseSum) != 0ull) {
-              raise(cur, ok, eacc);
-              e = exp_sum(cur, ok);
-            }
+            if (off(e)) e = raise(cur, ok, eacc);
             eacc += e;
             if constexpr (rg + 1 < NRG && !SG::PIPE) nxt = mma(qr[rg + 1], kf);
           });
@@ -1230,10 +1238,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
                 return b_scored && pos >= lo && pos < lq;
               };
               float e = exp_sum(sc, ok);
-              if (__ballot(e > kRaiseSum) != 0ull) {
-                raise(sc, ok, eacc);
-                e = exp_sum(sc, ok);
-              }
+              if (off(e)) e = raise(sc, ok, eacc);
               eacc += e;
             }
           });
@@ -1259,7 +1264,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
     float fw[4], emax = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      fw[w] = (xm[w] == neg_inf()) ? 0.f : exp2_fast(xm[w] - g);
+      fw[w] = (xm[w] == neg_inf()) ? 0.f : (MASK && xm[w] == g) ? 1.f : exp2_fast(xm[w] - g);
       emax = fmaxf(emax, wmx[w] * fw[w]);
     }
     kernarg_args fa = fresh();
@@ -1317,15 +1322,15 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
     const int64_t row = static_cast<int64_t>(h) * Nt + t;
     typedef __attribute__((address_space(1))) int32_t g_i32;
     typedef __attribute__((address_space(1))) uint8_t g_u8;
-    g_i32* ids = (g_i32*)(fa->ids + row * Nb);
-    g_i32* pids = (g_i32*)(fa->pids + row * Nb);
     g_u8* selo = fa->sel_out ? (g_u8*)(fa->sel_out + row * Nb) : nullptr;
-    if (!fa->ids) {  // the mask alone
+    if constexpr (MASK) {
       for (int base = w0, it = 0; base < w1; base += 64, ++it)
         if (base + lane < w1) selo[base + lane] = (selbits >> it) & 1u;
       for (int b = nvis + tid; b < Nb; b += kThreads) selo[b] = 0;
       continue;
     }
+    g_i32* ids = (g_i32*)(fa->ids + row * Nb);
+    g_i32* pids = (g_i32*)(fa->pids + row * Nb);
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (int base = w0, it = 0; base < w1; base += 64, ++it) {
       const int b = base + lane;
@@ -1525,6 +1530,13 @@ int dispatch_rows(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
   return check_launch("score_select");
 }
 
+template <typename T, int D, bool MASK>
+int launch_stream(bool swz, dim3 grid, hipStream_t stream, const SelectArgs& a) {
+  if constexpr (D == 64 || D == 128)
+    if (swz) return launch_with_lds(select_stream_kernel<T, D, true, MASK>, grid, stream_lds_bytes(a.Nb), stream, a);
+  return launch_with_lds(select_stream_kernel<T, D, false, MASK>, grid, stream_lds_bytes(a.Nb), stream, a);
+}
+
 template <typename T>
 int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a, bool* done) {
   *done = true;
@@ -1547,14 +1559,14 @@ int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
     // bits clear (q_rs * 2 a multiple of the row size)
     const int64_t rpi = 1024 / (D * 2);
     const bool swz = (D == 64 || D == 128) && a.tq % rpi == 0 && (a.q_rs * 2) % (D * 2) == 0;
+    const bool mask = a.ids == nullptr;
     switch (D) {
       case 64:
-        return swz ? launch_with_lds(select_stream_kernel<T, 64, true>, sgrid, stream_lds_bytes(a.Nb), stream, s)
-                   : launch_with_lds(select_stream_kernel<T, 64, false>, sgrid, stream_lds_bytes(a.Nb), stream, s);
-      case 96: return launch_with_lds(select_stream_kernel<T, 96, false>, sgrid, stream_lds_bytes(a.Nb), stream, s);
+        return mask ? launch_stream<T, 64, true>(swz, sgrid, stream, s) : launch_stream<T, 64, false>(swz, sgrid, stream, s);
+      case 96:
+        return mask ? launch_stream<T, 96, true>(swz, sgrid, stream, s) : launch_stream<T, 96, false>(swz, sgrid, stream, s);
       case 128:
-        return swz ? launch_with_lds(select_stream_kernel<T, 128, true>, sgrid, stream_lds_bytes(a.Nb), stream, s)
-                   : launch_with_lds(select_stream_kernel<T, 128, false>, sgrid, stream_lds_bytes(a.Nb), stream, s);
+        return mask ? launch_stream<T, 128, true>(swz, sgrid, stream, s) : launch_stream<T, 128, false>(swz, sgrid, stream, s);
       default: break;  // D = 256: the owner path below (its registers hold no resident Q)
     }
   }

@@ -94,3 +94,47 @@ def test_infinite_and_nan_queries_leave_other_tiles_alone(cuda):
     assert torch.equal(sel[:, [0, 3]], clean[:, [0, 3]])
     assert bool(scores[0, 0, 40].isnan().all()) and not bool(scores[0, 1, 70].isfinite().any())
     assert bool(scores[0, 0, 39].isfinite().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+@pytest.mark.parametrize("alpha", [0.0, 0.2])
+@pytest.mark.parametrize("poison", ["q inf", "q -inf", "q rows nan", "k nan", "k inf", "k -inf",
+                                    "q and k", "large"])
+def test_masks_of_infinities_and_nan_do_not_depend_on_the_scores(cuda, dtype, d, alpha, poison):
+    """The mask alone (the streaming kernel up to D = 128) is the mask that
+    comes with the scores (the row path) where logits are infinite or NaN, and
+    at 200 times the usual logits."""
+    inf = float("inf")
+    for heads, tq, bk, nb, qlen, offset in [((4, 1), 32, 16, 65, 333, 700),
+                                            ((6, 2), 40, 16, 33, 500, 20),
+                                            ((8, 2), 128, 128, 20, 2500, 0)]:
+        g = torch.Generator().manual_seed(d + nb)
+        q = torch.randn((heads[0], -(-qlen // tq) * tq, d), generator=g)
+        q[:, qlen:] = 0
+        pk = 0.7 * torch.randn((heads[1], nb, d), generator=g)
+        at = qlen // 2 + 3
+        if poison in ("q inf", "q and k"):
+            q[:, at:at + 40:7, 2] = inf
+            q[-1, at + 3, 5] = -inf
+        if poison == "q -inf":  # logits of -inf before a wave's first finite one
+            pk[:, :, 3] = pk[:, :, 3].abs() + 0.1
+            q[:, :qlen:3, 3] = -inf
+        if poison == "q rows nan":
+            q[:, at:at + 70] = float("nan")
+        if poison == "k nan":
+            pk[0, nb // 2, 1] = float("nan")
+        if poison in ("k inf", "q and k"):
+            pk[-1, nb // 2, 2] = inf
+        if poison == "k -inf":
+            pk[0, nb // 3, 4] = -inf
+        if poison == "large":
+            q, pk = 200 * q, 200 * pk
+        masks = []
+        for chunk in (None, 1):
+            config = FPV2Config(block_k=bk, tile_q=tq, alpha=alpha, sink_tokens=bk,
+                                window_tokens=2 * bk, last_n_blocks=1, score_chunk_tiles=chunk)
+            masks.append(block_scores_and_select(q.to(dtype).to(cuda), pk.to(dtype).to(cuda),
+                                                 scale=d ** -0.5, config=config, offset=offset,
+                                                 query_length=qlen)[0])
+        assert torch.equal(*masks), (heads, int((masks[0] != masks[1]).sum()))
