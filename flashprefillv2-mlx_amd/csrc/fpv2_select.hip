@@ -251,7 +251,11 @@ __device__ __forceinline__ void rows_mma(u32x4 q, u32x4 k, f32x16& acc) {
   }
 }
 
-template <typename T, int D>
+// WIDE: score rows by 64-bit addresses, for calls whose 32-row groups span more
+// scores than a buffer's 32-bit offsets reach (tile_q not a multiple of 32: a
+// group's rows belong to several query heads).  131072 tokens, four heads,
+// tile_q 16, D = 128: 0.83 ms (180 ms in the generic kernel).
+template <typename T, int D, bool WIDE>
 __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 : 2) <= 512 ? 2 : 1)) void select_rows_kernel(SelectArgs a) {
   constexpr int ES = std::is_same<T, float>::value ? 4 : 2;  // bytes per element
   constexpr int NF = D * ES / 32;  // fragments per row and lane half
@@ -304,17 +308,29 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
       }
       lo_pos = __builtin_amdgcn_readfirstlane(lo_pos);
       const bool full = lo_pos >= 0 && __builtin_amdgcn_readfirstlane(hi_pos) < lq;
-      // Score rows of the group, from the first one's (rows follow each
-      // other upwards: the padded length covers a tile): byte offsets of the
-      // 16 rows the lane's accumulators hold, rows (j/4)*8 + hf*4 + j%4.
-      const int score_row = static_cast<int>(g * a.Lq_pad) + pos;  // of the KV head (host-checked range)
-      const int score_row0 = __builtin_amdgcn_readfirstlane(score_row);
-      const rsrc_t sr = make_rsrc(a.scores + ((ti.h * a.G * a.Lq_pad) + score_row0) * a.Nb, 0x7fffffffu);
+      // Score rows of the group: of the 16 rows the lane's accumulators hold,
+      // (j/4)*8 + hf*4 + j%4, the byte offsets from the group's first row (rows
+      // follow each other upwards: the padded length covers a tile), or
+      // (WIDE) the addresses, null where there is no row.
+      rsrc_t sr;
       uint32_t srow[16];
-      if (a.scores) {
-        const uint32_t mine = pos >= 0 ? static_cast<uint32_t>(score_row - score_row0) * static_cast<uint32_t>(a.Nb) * 4u : kOOB;
+      float* wrow[16];
+      if constexpr (WIDE) {
+        const int64_t mine = pos >= 0 ? ti.h * a.G * a.Lq_pad + g * a.Lq_pad + pos : -1;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) srow[j] = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3)) + l32 * 4;
+        for (int j = 0; j < 16; ++j) {
+          const int64_t row = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3));
+          wrow[j] = row < 0 ? nullptr : a.scores + row * a.Nb + l32;
+        }
+      } else {
+        const int score_row = static_cast<int>(g * a.Lq_pad) + pos;  // of the KV head (host-checked range)
+        const int score_row0 = __builtin_amdgcn_readfirstlane(score_row);
+        sr = make_rsrc(a.scores + ((ti.h * a.G * a.Lq_pad) + score_row0) * a.Nb, 0x7fffffffu);
+        if (a.scores) {
+          const uint32_t mine = pos >= 0 ? static_cast<uint32_t>(score_row - score_row0) * static_cast<uint32_t>(a.Nb) * 4u : kOOB;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) srow[j] = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3)) + l32 * 4;
+        }
       }
       for (int c0 = 0; c0 < win_n; c0 += 32) {
         const int64_t b = win + c0 + l32;
@@ -331,7 +347,12 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
 #pragma unroll
           for (int k = 0; k < NF; ++k) rows_mma<T>(qf[k], kf[k], acc);
         }
-        if (a.scores && b < a.Nb) {
+        if (WIDE && b < a.Nb) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (wrow[j]) wrow[j][win + c0] = acc[j] * a.scale;
+        }
+        if (!WIDE && a.scores && b < a.Nb) {
           const uint32_t at = static_cast<uint32_t>(win + c0) * 4u;
 #pragma unroll
           for (int j = 0; j < 16; ++j)
@@ -1495,18 +1516,20 @@ int launch_generic(K kernel, dim3 grid, size_t lds, hipStream_t stream, const Se
   return check_launch("score_select");
 }
 
+template <typename T, int D>
+int launch_rows(bool wide, dim3 grid, hipStream_t stream, const SelectArgs& a) {
+  return wide ? launch_with_lds(select_rows_kernel<T, D, true>, grid, rows_lds_bytes(a.Nb), stream, a)
+              : launch_with_lds(select_rows_kernel<T, D, false>, grid, rows_lds_bytes(a.Nb), stream, a);
+}
+
 template <typename T>
 int dispatch_rows(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a, bool* done) {
-  // score rows of a head and the byte offsets of a 32-row group's rows in 32
-  // bits (the generic kernel serves the rest)
+  // whether a head's score rows and the byte offsets of a 32-row group's rows
+  // pass 32 bits
   const int64_t heads = a.tq >= 32 ? 2 : 32 / a.tq + 2;  // query heads a row group touches
-  if (a.scores && (a.G * a.Lq_pad >= (1LL << 31) ||
-                   (a.G > 1 && a.tq % 32 ? heads * a.Lq_pad : 32) * a.Nb * 4 >= kMaxRsrcBytes)) {
-    *done = false;
-    return 0;
-  }
+  const bool wide = a.scores && (a.G * a.Lq_pad >= (1LL << 31) ||
+                                 (a.G > 1 && a.tq % 32 ? heads * a.Lq_pad : 32) * a.Nb * 4 >= kMaxRsrcBytes);
   *done = true;
-  const size_t lds = rows_lds_bytes(a.Nb);
   SelectArgs s = a;
   const dim3 tiles = grid;
   const int parts = a.parts ? rows_parts(tiles.x, a.G * a.tq) : 1;
@@ -1514,10 +1537,10 @@ int dispatch_rows(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
   if (parts == 1) s.parts = nullptr;
   int rc;
   switch (D) {
-    case 64: rc = launch_with_lds(select_rows_kernel<T, 64>, grid, lds, stream, s); break;
-    case 96: rc = launch_with_lds(select_rows_kernel<T, 96>, grid, lds, stream, s); break;
-    case 128: rc = launch_with_lds(select_rows_kernel<T, 128>, grid, lds, stream, s); break;
-    case 256: rc = launch_with_lds(select_rows_kernel<T, 256>, grid, lds, stream, s); break;
+    case 64: rc = launch_rows<T, 64>(wide, grid, stream, s); break;
+    case 96: rc = launch_rows<T, 96>(wide, grid, stream, s); break;
+    case 128: rc = launch_rows<T, 128>(wide, grid, stream, s); break;
+    case 256: rc = launch_rows<T, 256>(wide, grid, stream, s); break;
     default: *done = false; return 0;
   }
   if (rc || parts == 1) return rc;

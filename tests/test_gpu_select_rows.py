@@ -138,3 +138,50 @@ def test_masks_of_infinities_and_nan_do_not_depend_on_the_scores(cuda, dtype, d,
                                                  scale=d ** -0.5, config=config, offset=offset,
                                                  query_length=qlen)[0])
         assert torch.equal(*masks), (heads, int((masks[0] != masks[1]).sum()))
+
+
+def _scored(cuda, q, pk, config, repeat=3):
+    """(mask, scores, least milliseconds) of a call with its raw scores."""
+    best = float("inf")
+    for _ in range(repeat):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        sel, scores = block_scores_and_select(q, pk, scale=q.shape[-1] ** -0.5, config=config)
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end))
+    return sel, scores, best
+
+
+@pytest.mark.parametrize(("dtype", "heads", "tq", "length", "nb"), [
+    (torch.bfloat16, 4, 16, 16384, 8192),  # two heads a row group, sixteen windows of blocks
+    (torch.float16, 3, 40, 131080, 2049),  # groups that end and begin inside heads
+    (torch.float32, 4, 16, 16384, 8192),
+])
+def test_row_groups_over_2_gib_of_scores(cuda, dtype, heads, tq, length, nb):
+    """Row groups whose rows lie 2 GiB of scores and more apart are served by
+    the same kernel with 64-bit addresses: scores of rows all over the call
+    against float64, mask against the mask alone, and no slower than a call of
+    a quarter of the scores by more than twice the work (the kernel that takes
+    one thread per block was 250 times slower)."""
+    d = 64
+    g = torch.Generator(device=cuda).manual_seed(heads)
+    q = torch.randn((heads, length, d), generator=g, device=cuda).to(dtype)
+    pk = (0.7 * torch.randn((1, nb, d), generator=g, device=cuda)).to(dtype)
+    block = -(-length // nb)
+    config = FPV2Config(block_k=block, tile_q=tq, alpha=0.2, sink_tokens=block, window_tokens=block)
+    assert (32 // tq + 2) * length * nb * 4 >= 2 ** 31
+    sel, scores, ms = _scored(cuda, q, pk, config)
+    alone, _ = block_scores_and_select(q, pk, scale=d ** -0.5, config=FPV2Config(
+        **{**config.__dict__, "score_chunk_tiles": 1}))
+    # (energies round to either side of alpha: a few flags of millions)
+    assert int((sel != alone).sum()) <= 1e-4 * sel.numel()
+    rows = torch.randint(0, length, (200,), generator=g, device=cuda)
+    rows[:4] = torch.tensor([0, tq - 1, tq, length - 1])
+    want = q[:, rows].double() @ pk[0].double().T * d ** -0.5
+    mass = q[:, rows].double().abs() @ pk[0].double().abs().T * d ** -0.5
+    assert bool(((scores[0][:, rows].double() - want).abs() <= (d + 2) * 2.0 ** -24 * mass).all())
+    del scores, want, mass
+    quarter = -(-length // 4 // tq) * tq
+    _, _, ms4 = _scored(cuda, q[:, :quarter].contiguous(), pk, config)
+    assert ms < 8 * ms4 + 0.2
