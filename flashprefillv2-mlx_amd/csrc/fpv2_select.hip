@@ -206,9 +206,9 @@ __device__ void finish_tile(const SelectArgs& a, const TileInfo& ti, float* cb, 
 
 // ---------------------------------------------------------------------------
 // Row path: 16-bit or float32 queries and pooled keys, D in {64, 96, 128,
-// 256}, taken when the caller asks for the scores or for the mask alone, when
-// the scale is not positive and for float32 (the streaming and owner paths
-// below serve the rest).  Each wave owns 32-row groups of the tile and
+// 256}, taken when the caller asks for the scores, when the scale is not
+// positive, for float32, and for masks that the streaming and owner paths
+// below do not serve (D = 256 with few blocks; sizes past 32 bits).  Each wave owns 32-row groups of the tile and
 // multiplies them with every chunk of 32 pooled keys, both read straight into
 // MFMA fragments (the keys of a head stay in L2): S = Q . Kbar^T, a lane
 // holding 16 rows of one block, from which scores are stored 128 contiguous
@@ -505,6 +505,8 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 // [w * span, (w + 1) * span) 64 at a time with ballots: one pass counts, the
 // waves' counts are exchanged through LDS, a second pass writes each block's
 // positions (selected ascending, then the rest ascending; likewise pruned).
+// MASK: the mask alone.
+template <bool MASK>
 __device__ __forceinline__ void finish_lists(const SelectArgs& a, int h, int t, int tile_first, int tile_last,
                             int nfv, const float* eb, float* fred, int* ired) {
   const int tid = threadIdx.x;
@@ -531,6 +533,15 @@ __device__ __forceinline__ void finish_lists(const SelectArgs& a, int h, int t, 
     sel = (E >= thr || forced) && bs <= tile_last;
     pru = !sel && min(be, lk) <= tile_first;
   };
+  if constexpr (MASK) {
+    uint8_t* const selo = a.sel_out + (static_cast<int64_t>(h) * a.Nt + t) * a.Nb;
+    for (int b = tid; b < Nb; b += kThreads) {
+      bool sel, pru;
+      flags(b, sel, pru);
+      selo[b] = sel;
+    }
+    return;
+  }
   const int span = ((Nb + 4 * 64 - 1) / (4 * 64)) * 64;
   const int w0 = min(Nb, wave * span), w1 = min(Nb, w0 + span);
   int ns = 0, np = 0;
@@ -611,7 +622,8 @@ constexpr size_t own_lds_bytes(int64_t Nb) {
 constexpr float kRaiseSum = 65536.f;  // 2^kWaveSlack
 static_assert(kWaveSlack == 16.f, "kRaiseSum is 2^kWaveSlack");
 
-template <typename T, int D>
+// MASK: the mask alone, as the streaming kernel's.
+template <typename T, int D, bool MASK>
 __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) void select_own_kernel(SelectArgs a) {
   constexpr int KS = D / 16;  // MFMA k-steps over the head dimension
   constexpr int LDQ = D + 8;
@@ -709,15 +721,21 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
     float lm = neg_inf();
 #pragma unroll
     for (int j = 0; j < 16; ++j) lm = ok(j) ? fmaxf(lm, s[j]) : lm;
-    const float m_new = wave_max_any(lm) * sc2;
-    const float f = (mref == neg_inf()) ? 0.f : exp2_fast(mref - m_new);
+    const float top = wave_max_any(lm) * sc2;
+    // (MASK: also entered for a NaN sum, whose wave may need no raise)
+    const float m_new = MASK ? fmaxf(mref, top) : top;
+    const float f = (mref == neg_inf()) ? 0.f : (MASK && mref == m_new) ? 1.f : exp2_fast(mref - m_new);
     eacc *= f;
     for (int cc = wave; cc < nchunks; cc += 4) {
       const int bb = cc * 32 + l32;
       if (hf == 0 && bb < nfv) eb[bb] *= f;
     }
     mref = m_new;
+    const float e = exp_sum(s, ok);
+    return MASK && lm == neg_inf() ? 0.f : e;
   };
+  // whether the sum needs another reference (MASK: or is NaN)
+  auto off = [](float e) { return __ballot(MASK ? !(e <= kRaiseSum) : e > kRaiseSum) != 0ull; };
 
   for (int64_t rc = 0; rc < R; rc += kRowsPerPass) {
     __syncthreads();  // the previous pass is done with qs, qoff and rpos
@@ -829,10 +847,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
             __builtin_amdgcn_sched_group_barrier(0x002, 48 / KS, 0);
           }
         }
-        if (__ballot(e > kRaiseSum) != 0ull) {
-          raise(cur, ok, eacc);
-          e = exp_sum(cur, ok);
-        }
+        if (off(e)) e = raise(cur, ok, eacc);
         eacc += e;
         if constexpr (rg + 1 < 4 && !kResident) nxt = rg_scores(std::integral_constant<int, rg + 1>{}, kf);
       });
@@ -857,10 +872,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
           }
           auto ok = [&](int j) { return okr[j]; };
           float e = exp_sum(s, ok);
-          if (__ballot(e > kRaiseSum) != 0ull) {
-            raise(s, ok, eacc);
-            e = exp_sum(s, ok);
-          }
+          if (off(e)) e = raise(s, ok, eacc);
           eacc += e;
         }
       });
@@ -883,13 +895,13 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(1, 
   if (lane == 0) xm[wave] = mref;
   __syncthreads();
   const float g = fmaxf(fmaxf(xm[0], xm[1]), fmaxf(xm[2], xm[3]));
-  const float f = (mref == neg_inf()) ? 0.f : exp2_fast(mref - g);
+  const float f = (mref == neg_inf()) ? 0.f : (MASK && mref == g) ? 1.f : exp2_fast(mref - g);
   for (int cc = wave; cc < nchunks; cc += 4) {
     const int bb = cc * 32 + l32;
     if (hf == 0 && bb < nfv) eb[bb] *= f;
   }
   __syncthreads();
-  finish_lists(a, static_cast<int>(ti.h), static_cast<int>(ti.t), static_cast<int>(ti.tile_first),
+  finish_lists<MASK>(a, static_cast<int>(ti.h), static_cast<int>(ti.t), static_cast<int>(ti.tile_first),
               static_cast<int>(ti.tile_last), nfv, eb, fred, ired);
 }
 
@@ -1593,14 +1605,21 @@ int dispatch_mfma(int64_t D, dim3 grid, hipStream_t stream, const SelectArgs& a,
       default: break;  // D = 256: the owner path below (its registers hold no resident Q)
     }
   }
-  if (a.scores == nullptr && a.scale > 0.f && a.ids != nullptr && small) {
-    switch (D) {
-      case 64: return launch_with_lds(select_own_kernel<T, 64>, grid, own_lds_bytes<64>(a.Nb), stream, a);
-      case 96: return launch_with_lds(select_own_kernel<T, 96>, grid, own_lds_bytes<96>(a.Nb), stream, a);
-      case 128: return launch_with_lds(select_own_kernel<T, 128>, grid, own_lds_bytes<128>(a.Nb), stream, a);
-      case 256: return launch_with_lds(select_own_kernel<T, 256>, grid, own_lds_bytes<256>(a.Nb), stream, a);
-
-      default: break;
+  if (a.scores == nullptr && a.scale > 0.f && small) {
+    if (a.ids != nullptr) {
+      switch (D) {
+        case 64: return launch_with_lds(select_own_kernel<T, 64, false>, grid, own_lds_bytes<64>(a.Nb), stream, a);
+        case 96: return launch_with_lds(select_own_kernel<T, 96, false>, grid, own_lds_bytes<96>(a.Nb), stream, a);
+        case 128: return launch_with_lds(select_own_kernel<T, 128, false>, grid, own_lds_bytes<128>(a.Nb), stream, a);
+        case 256: return launch_with_lds(select_own_kernel<T, 256, false>, grid, own_lds_bytes<256>(a.Nb), stream, a);
+        default: break;
+      }
+    } else if (a.sel_out != nullptr && D == 256 && a.Nb >= (a.G * a.tq >= 128 ? 64 : 128)) {
+      // Masks at D = 256, row path / here: 32 / 8 heads, 64 blocks 41 / 33 us,
+      // 1024 blocks 4022 / 1375 us; 2048 queries of one KV head behind 1024
+      // blocks 67 / 26 us; but 16 blocks 16 / 22 us, and 64 blocks at 32 rows
+      // a tile 23 / 27 us.
+      return launch_with_lds(select_own_kernel<T, 256, true>, grid, own_lds_bytes<256>(a.Nb), stream, a);
     }
   }
   return dispatch_rows<T>(D, grid, stream, a, done);

@@ -74,6 +74,16 @@ def test_windows_of_blocks(cuda, dtype, nb):
     _check(cuda, dtype, 64, (4, 2), 32, nb, 90, nb * 4 - 130, 4)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("d", "heads", "tq", "nb", "qlen"), [
+    (256, (4, 1), 32, 64, 100),  # the mask alone from the owner kernel
+    (256, (4, 1), 40, 70, 100),  # its second pass of rows
+    (256, (2, 1), 40, 130, 90),  # fewer rows than a pass
+])
+def test_masks_of_the_owner_kernel(cuda, dtype, d, heads, tq, nb, qlen):
+    _check(cuda, dtype, d, heads, tq, nb, qlen, 4 * nb - qlen - 3, 4)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("sign", [-1.0, 0.0])
 def test_scales_that_are_not_positive(cuda, dtype, sign):
@@ -102,9 +112,9 @@ def test_infinite_and_nan_queries_leave_other_tiles_alone(cuda):
 @pytest.mark.parametrize("poison", ["q inf", "q -inf", "q rows nan", "k nan", "k inf", "k -inf",
                                     "q and k", "large"])
 def test_masks_of_infinities_and_nan_do_not_depend_on_the_scores(cuda, dtype, d, alpha, poison):
-    """The mask alone (the streaming kernel up to D = 128) is the mask that
-    comes with the scores (the row path) where logits are infinite or NaN, and
-    at 200 times the usual logits."""
+    """The mask alone (the streaming kernel up to D = 128, the owner kernel for
+    the 65 blocks of D = 256) is the mask that comes with the scores (the row
+    path) where logits are infinite or NaN, and at 200 times the usual logits."""
     inf = float("inf")
     for heads, tq, bk, nb, qlen, offset in [((4, 1), 32, 16, 65, 333, 700),
                                             ((6, 2), 40, 16, 33, 500, 20),
