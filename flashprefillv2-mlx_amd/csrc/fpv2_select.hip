@@ -35,6 +35,7 @@ struct SelectArgs {
   int32_t* pcounts;
   uint32_t tq_magic;  // ceil(2^32 / tq), streaming path
   float* parts;  // row path in parts: [tile][part][c, e][Nb]
+  int row_waves;  // row path: waves side by side on the rows (1, 2 or 4)
 };
 
 struct TileInfo {
@@ -208,22 +209,23 @@ __device__ void finish_tile(const SelectArgs& a, const TileInfo& ti, float* cb, 
 // Row path: 16-bit or float32 queries and pooled keys, D in {64, 96, 128,
 // 256}, taken when the caller asks for the scores, when the scale is not
 // positive, for float32, and for masks that the streaming and owner paths
-// below do not serve (D = 256 with few blocks; sizes past 32 bits).  Each wave owns 32-row groups of the tile and
-// multiplies them with every chunk of 32 pooled keys, both read straight into
-// MFMA fragments (the keys of a head stay in L2): S = Q . Kbar^T, a lane
-// holding 16 rows of one block, from which scores are stored 128 contiguous
-// bytes per row.  Row groups rather than chunks are split over the waves so
-// that short prompts, whose blocks make only one or two chunks, keep every
-// wave busy.  The blocks pass in windows of kRowsWin; each wave sums its own
-// (c, e) per block of the window in LDS, and the waves' pairs are merged at its
-// end.  float32 uses v_mfma_f32_32x32x2_f32: the products and sums stay in
-// float32.
+// below do not serve (D = 256 with few blocks; sizes past 32 bits).  Each wave
+// holds RG 32-row groups of the tile and multiplies them with chunks of 32
+// pooled keys, both read straight into MFMA fragments (the keys of a head stay
+// in L2): S = Q . Kbar^T, a lane holding 16 rows of one block, from which
+// scores are stored 128 contiguous bytes per row.  Rows before chunks are split
+// over the waves, so that short prompts, whose blocks make only one or two
+// chunks, keep every wave busy, and waves on the same chunk share its read;
+// row_waves of them are on the rows, the others on other chunks of the same
+// rows (launch_rows).  The blocks pass in windows of kRowsWin; each wave sums
+// its own (c, e) per block of the window in LDS, and the waves' pairs are
+// merged at its end.  float32 uses v_mfma_f32_32x32x2_f32: the products and
+// sums stay in float32.
 //   Bound by latency (loads of Q, then of each chunk) and, with scores, by
-// their stores.  Measured at D = 128: 8192 tokens, 32 / 8 heads, bfloat16 with
-// scores 33 us (67 us with one wave per chunk; 134 MB, 27 us at the rate of a
-// copy); 5000 tokens, 8 / 2 heads, float32 24 us (34 us with whole tiles; 4960 us
-// without MFMA, one thread per block); the mask alone at 15000 tokens 68 us (96 us; the
-// streaming path takes 45 us and serves it where it can).
+// their stores.  Measured at D = 128 (calls): 8192 tokens, 32 / 8 heads,
+// bfloat16 with scores 29 us (65 us with one wave per chunk and Q in LDS; 134
+// MB, 27 us at the rate of a copy); 5000 tokens, 8 / 2 heads, float32 24 us (34
+// us with whole tiles; 4960 us without MFMA, one thread per block).
 //   Where the call has fewer tiles than the chip holds workgroups and the
 // caller gives a workspace, a tile's row groups are dealt to gridDim.y
 // workgroups (rows_parts): each leaves its (c, e) per block in a.parts, and
@@ -254,11 +256,12 @@ __device__ __forceinline__ void rows_mma(u32x4 q, u32x4 k, f32x16& acc) {
 // WIDE: score rows by 64-bit addresses, for calls whose 32-row groups span more
 // scores than a buffer's 32-bit offsets reach (tile_q not a multiple of 32: a
 // group's rows belong to several query heads).  131072 tokens, four heads,
-// tile_q 16, D = 128: 0.83 ms (180 ms in the generic kernel).
-template <typename T, int D, bool WIDE>
+// tile_q 16, D = 128: 0.71 ms (180 ms in the generic kernel).
+template <typename T, int D, int RG, bool WIDE>
 __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 : 2) <= 512 ? 2 : 1)) void select_rows_kernel(SelectArgs a) {
   constexpr int ES = std::is_same<T, float>::value ? 4 : 2;  // bytes per element
   constexpr int NF = D * ES / 32;  // fragments per row and lane half
+  constexpr int WR = RG * 32;      // rows a wave holds
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ float fred[4];
   __shared__ int ired[8];
@@ -278,6 +281,9 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
   const unsigned char* qh = static_cast<const unsigned char*>(a.q) + ti.h * a.G * a.q_hs * ES;
   const float sc2 = a.scale * kLog2e;
   const int lq = static_cast<int>(a.Lq);
+  // nr waves on the rows, times nc on the chunks
+  const int nr = a.row_waves, nc = nr == 4 ? 1 : nr == 2 ? 2 : 4;
+  const int wr = wave & (nr - 1), wk = nr == 4 ? 0 : nr == 2 ? wave >> 1 : wave;
 
   for (int64_t win = 0; win < n_comp; win += kRowsWin) {
     const int win_n = static_cast<int>(n_comp - win < kRowsWin ? n_comp - win : kRowsWin);
@@ -285,110 +291,123 @@ __global__ __launch_bounds__(kThreads, (D * (std::is_same<T, float>::value ? 4 :
       wc[i] = neg_inf();
       we[i] = 0.f;
     }
-    for (int64_t rc = blockIdx.y * kRowsPerPass + wave * 32; rc < R; rc += gridDim.y * kRowsPerPass) {
-      // this lane's query row (zeros past the tile or the valid length)
-      const int64_t pr = rc + l32;
-      const int64_t g = pr / a.tq;
-      const int pos = pr < R ? static_cast<int>(ti.t * a.tq + (pr - g * a.tq)) : -1;
-      u32x4 qf[NF];
-#pragma unroll
-      for (int k = 0; k < NF; ++k) qf[k] = u32x4{0u, 0u, 0u, 0u};
-      if (pos >= 0 && pos < lq) {
-        const unsigned char* src = qh + (g * a.q_hs + static_cast<int64_t>(pos) * a.q_rs) * ES + hf * 16;
-#pragma unroll
-        for (int k = 0; k < NF; ++k) qf[k] = load16(src + k * 32);
-      }
-      // (wave-uniform) lowest position, and whether every row is present and
-      // inside the valid length
-      int lo_pos = pos, hi_pos = pos;
-#pragma unroll
-      for (int o = 16; o >= 1; o >>= 1) {
-        lo_pos = min(lo_pos, __shfl_xor(lo_pos, o));
-        hi_pos = max(hi_pos, __shfl_xor(hi_pos, o));
-      }
-      lo_pos = __builtin_amdgcn_readfirstlane(lo_pos);
-      const bool full = lo_pos >= 0 && __builtin_amdgcn_readfirstlane(hi_pos) < lq;
-      // Score rows of the group: of the 16 rows the lane's accumulators hold,
-      // (j/4)*8 + hf*4 + j%4, the byte offsets from the group's first row (rows
-      // follow each other upwards: the padded length covers a tile), or
+    for (int64_t rc = static_cast<int64_t>(blockIdx.y * nr + wr) * WR; rc < R; rc += gridDim.y * nr * WR) {
+      u32x4 qf[RG][NF];
+      int pos[RG], lo_pos[RG];
+      bool full[RG];
+      // Score rows of a 32-row group: of the 16 rows the lane's accumulators
+      // hold, (j/4)*8 + hf*4 + j%4, the byte offsets from the group's first row
+      // (rows follow each other upwards: the padded length covers a tile), or
       // (WIDE) the addresses, null where there is no row.
-      rsrc_t sr;
-      uint32_t srow[16];
-      float* wrow[16];
-      if constexpr (WIDE) {
-        const int64_t mine = pos >= 0 ? ti.h * a.G * a.Lq_pad + g * a.Lq_pad + pos : -1;
+      rsrc_t sr[RG];
+      uint32_t srow[RG][16];
+      float* wrow[RG][16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int64_t row = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3));
-          wrow[j] = row < 0 ? nullptr : a.scores + row * a.Nb + l32;
+      for (int rg = 0; rg < RG; ++rg) {
+        // this lane's query row (zeros past the tile or the valid length)
+        const int64_t pr = rc + rg * 32 + l32;
+        const int64_t g = pr / a.tq;
+        pos[rg] = pr < R ? static_cast<int>(ti.t * a.tq + (pr - g * a.tq)) : -1;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) qf[rg][k] = u32x4{0u, 0u, 0u, 0u};
+        if (pos[rg] >= 0 && pos[rg] < lq) {
+          const unsigned char* src = qh + (g * a.q_hs + static_cast<int64_t>(pos[rg]) * a.q_rs) * ES + hf * 16;
+#pragma unroll
+          for (int k = 0; k < NF; ++k) qf[rg][k] = load16(src + k * 32);
         }
-      } else {
-        const int score_row = static_cast<int>(g * a.Lq_pad) + pos;  // of the KV head (host-checked range)
-        const int score_row0 = __builtin_amdgcn_readfirstlane(score_row);
-        sr = make_rsrc(a.scores + ((ti.h * a.G * a.Lq_pad) + score_row0) * a.Nb, 0x7fffffffu);
-        if (a.scores) {
-          const uint32_t mine = pos >= 0 ? static_cast<uint32_t>(score_row - score_row0) * static_cast<uint32_t>(a.Nb) * 4u : kOOB;
+        // (wave-uniform) lowest position, and whether every row is present
+        // and inside the valid length
+        int lo = pos[rg], hi = pos[rg];
 #pragma unroll
-          for (int j = 0; j < 16; ++j) srow[j] = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3)) + l32 * 4;
+        for (int o = 16; o >= 1; o >>= 1) {
+          lo = min(lo, __shfl_xor(lo, o));
+          hi = max(hi, __shfl_xor(hi, o));
+        }
+        lo_pos[rg] = __builtin_amdgcn_readfirstlane(lo);
+        full[rg] = lo_pos[rg] >= 0 && __builtin_amdgcn_readfirstlane(hi) < lq;
+        if constexpr (WIDE) {
+          const int64_t mine = pos[rg] >= 0 ? ti.h * a.G * a.Lq_pad + g * a.Lq_pad + pos[rg] : -1;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int64_t row = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3));
+            wrow[rg][j] = row < 0 ? nullptr : a.scores + row * a.Nb + l32;
+          }
+        } else {
+          const int score_row = static_cast<int>(g * a.Lq_pad) + pos[rg];  // of the KV head (host-checked range)
+          const int score_row0 = __builtin_amdgcn_readfirstlane(score_row);
+          sr[rg] = make_rsrc(a.scores + ((ti.h * a.G * a.Lq_pad) + score_row0) * a.Nb, 0x7fffffffu);
+          if (a.scores) {
+            const uint32_t mine = pos[rg] >= 0 ? static_cast<uint32_t>(score_row - score_row0) * static_cast<uint32_t>(a.Nb) * 4u : kOOB;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) srow[rg][j] = __shfl(mine, (j >> 2) * 8 + hf * 4 + (j & 3)) + l32 * 4;
+          }
         }
       }
-      for (int c0 = 0; c0 < win_n; c0 += 32) {
+      for (int c0 = wk * 32; c0 < win_n; c0 += nc * 32) {
         const int64_t b = win + c0 + l32;
-        f32x16 acc = {};
-        {
-          u32x4 kf[NF];
+        u32x4 kf[NF];
 #pragma unroll
-          for (int k = 0; k < NF; ++k) kf[k] = u32x4{0u, 0u, 0u, 0u};
-          if (b < a.Nb) {
-            const unsigned char* src = pk + b * D * ES + hf * 16;
+        for (int k = 0; k < NF; ++k) kf[k] = u32x4{0u, 0u, 0u, 0u};
+        if (b < a.Nb) {
+          const unsigned char* src = pk + b * D * ES + hf * 16;
 #pragma unroll
-            for (int k = 0; k < NF; ++k) kf[k] = load16(src + k * 32);
-          }
-#pragma unroll
-          for (int k = 0; k < NF; ++k) rows_mma<T>(qf[k], kf[k], acc);
+          for (int k = 0; k < NF; ++k) kf[k] = load16(src + k * 32);
         }
-        if (WIDE && b < a.Nb) {
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (wrow[j]) wrow[j][win + c0] = acc[j] * a.scale;
-        }
-        if (!WIDE && a.scores && b < a.Nb) {
-          const uint32_t at = static_cast<uint32_t>(win + c0) * 4u;
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[j] * a.scale), sr, srow[j], at, 0);
-        }
-        if (win + c0 >= ti.nfv) continue;  // (uniform) no block of the chunk is scored
         // Rows that see block b (fully visible blocks only): from local
         // position lo; the others count as -inf.
         const int64_t lo64 = b * a.bk - a.offset;
         const int lo = lo64 < 0 ? 0 : static_cast<int>(lo64 > 0x7fffffff ? 0x7fffffff : lo64);
         const bool scored = b < ti.nfv;
-        float lm = neg_inf();
-        if (full && __ballot(scored && lo_pos < lo) == 0ull) {
+        float lm = neg_inf(), e = 0.f;
 #pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            acc[j] = scored ? acc[j] * sc2 : neg_inf();
-            lm = fmaxf(lm, acc[j]);
+        for (int rg = 0; rg < RG; ++rg) {
+          if (RG > 1 && rc + rg * 32 >= R) continue;  // (uniform) no such rows
+          f32x16 acc = {};
+#pragma unroll
+          for (int k = 0; k < NF; ++k) rows_mma<T>(qf[rg][k], kf[k], acc);
+          if (WIDE && b < a.Nb) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+              if (wrow[rg][j]) wrow[rg][j][win + c0] = acc[j] * a.scale;
           }
-        } else {
+          if (!WIDE && a.scores && b < a.Nb) {
+            const uint32_t at = static_cast<uint32_t>(win + c0) * 4u;
 #pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const int p = __shfl(pos, (j >> 2) * 8 + hf * 4 + (j & 3));
-            acc[j] = scored && p >= lo && p < lq ? acc[j] * sc2 : neg_inf();
-            lm = fmaxf(lm, acc[j]);
+            for (int j = 0; j < 16; ++j)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[j] * a.scale), sr[rg], srow[rg][j], at, 0);
+          }
+          if (win + c0 >= ti.nfv) continue;  // (uniform) no block of the chunk is scored
+          float gm = neg_inf();
+          if (full[rg] && __ballot(scored && lo_pos[rg] < lo) == 0ull) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+              acc[j] = scored ? acc[j] * sc2 : neg_inf();
+              gm = fmaxf(gm, acc[j]);
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+              const int p = __shfl(pos[rg], (j >> 2) * 8 + hf * 4 + (j & 3));
+              acc[j] = scored && p >= lo && p < lq ? acc[j] * sc2 : neg_inf();
+              gm = fmaxf(gm, acc[j]);
+            }
+          }
+          float ge = 0.f;
+          if (gm != neg_inf()) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) ge += exp2_fast(acc[j] - gm);
+          }
+          const float oc = __shfl_xor(gm, 32);
+          const float oe = __shfl_xor(ge, 32);
+          merge_ce(gm, ge, oc, oe);
+          if (rg == 0) {
+            lm = gm;
+            e = ge;
+          } else {
+            merge_ce(lm, e, gm, ge);
           }
         }
-        float e = 0.f;
-        if (lm != neg_inf()) {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) e += exp2_fast(acc[j] - lm);
-        }
-        // the other half of the wave holds the other 16 rows of the group
-        const float oc = __shfl_xor(lm, 32);
-        const float oe = __shfl_xor(e, 32);
-        merge_ce(lm, e, oc, oe);
-        if (hf == 0 && c0 + l32 < win_n) {
+        if (hf == 0 && win + c0 < ti.nfv && c0 + l32 < win_n) {
           float c = wc[c0 + l32], s = we[c0 + l32];
           merge_ce(c, s, lm, e);
           wc[c0 + l32] = c;
@@ -1528,10 +1547,50 @@ int launch_generic(K kernel, dim3 grid, size_t lds, hipStream_t stream, const Se
   return check_launch("score_select");
 }
 
+// How a tile's rows and chunks are dealt to the waves, by the tile's rows R and
+// the size of the head's pooled keys.  A wave that holds 64 rows reads each
+// chunk half as often as one that holds 32; waves on other chunks of the same
+// rows keep tiles of few rows from leaving waves idle, but share no reads.
+// With scores at D = 128, 32 rows and every wave on the rows / this rule:
+//   One chunk (up to 32 blocks): 32 rows a wave.  R = 256: 13.0 us (13.9 by 64
+//     rows).
+//   R >= 256: 64 rows a wave.  32 / 8 heads at 8k 32 / 29 us, 32k 383 / 297 us,
+//     64k 1407 / 1017 us; 16 / 8 heads (R = 256), 1024 blocks, 697 / 560 us.
+//   R in (64, 256): 64 rows a wave from kRowsKeys elements of keys on.  32k
+//     tokens, 1024 blocks, R = 96 / 128 / 160 / 192: 1076 / 955, 670 / 518 (one
+//     KV head), 1799 / 1516, 2857 / 2308 us; at 192 and 252 blocks R = 128 takes 67 /
+//     62 and 115 / 96 us, at 128 blocks 53 / 51 us for R = 128 but 47 / 48 us
+//     for R = 96 (16k: 127 / 138 us).  D = 64, R = 128: 288 blocks 103 / 106 us, 378
+//     blocks 257 / 222 us.
+//   R in (32, 64]: from twice as much.  D = 128: 288 blocks 83 / 88 us, 378
+//     blocks 124 / 114 us; D = 64: 378 blocks 85 / 94 us.
+//   32 rows a wave: all waves on the rows (idle ones where R < 97) while the
+//     chunks are few, since each wave loads its rows of Q first; two on the
+//     chunks from 64 blocks on for R <= 32 (R = 16, 64 blocks 36 / 32 us) and from
+//     128 for R <= 64 (35.4 / 33.9 us, but 40 blocks 15.6 / 16.5 us), four from 256
+//     on for R <= 32 (R = 16: 252 blocks 56 us, 60 by two; 192 blocks 52, 51 by
+//     two; 1024 blocks 934 / 652 us).
+// (128-row waves spill; float32 and D = 256 hold 32 rows at most, and so do
+// WIDE calls, where 64 at D = 64 are slower, 501 / 584 us.)
+constexpr int64_t kRowsKeys = 24000;
+
 template <typename T, int D>
-int launch_rows(bool wide, dim3 grid, hipStream_t stream, const SelectArgs& a) {
-  return wide ? launch_with_lds(select_rows_kernel<T, D, true>, grid, rows_lds_bytes(a.Nb), stream, a)
-              : launch_with_lds(select_rows_kernel<T, D, false>, grid, rows_lds_bytes(a.Nb), stream, a);
+int launch_rows(bool wide, dim3 grid, hipStream_t stream, SelectArgs a) {
+  const int64_t R = a.G * a.tq, keys = a.Nb * D;
+  const size_t lds = rows_lds_bytes(a.Nb);
+  if constexpr (!std::is_same<T, float>::value && D <= 128) {
+    if (!wide && grid.y == 1 && a.Nb > 32 && (R >= 256 || (R > 32 && keys >= (R > 64 ? kRowsKeys : 2 * kRowsKeys)))) {
+      const int64_t n = (R + 63) / 64;  // 64-row turns of the tile
+      // (four waves unless a fifth of their turns would be idle: R = 288, 2008
+      // blocks, 2502 us by four and 2340 us by two)
+      a.row_waves = R >= 256 && (keys < kRowsKeys || 16 * ((n + 3) / 4) <= 5 * n) ? 4 : n > 1 ? 2 : 1;
+      return launch_with_lds(select_rows_kernel<T, D, 2, false>, grid, lds, stream, a);
+    }
+  }
+  const int64_t n = (R + 31) / 32;
+  a.row_waves = n > 2 || a.Nb < (n > 1 ? 128 : 64) ? 4 : n > 1 || a.Nb < 256 ? 2 : 1;
+  return wide ? launch_with_lds(select_rows_kernel<T, D, 1, true>, grid, lds, stream, a)
+              : launch_with_lds(select_rows_kernel<T, D, 1, false>, grid, lds, stream, a);
 }
 
 template <typename T>

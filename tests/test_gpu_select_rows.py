@@ -76,6 +76,21 @@ def test_windows_of_blocks(cuda, dtype, nb):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize(("d", "heads", "tq", "nb", "qlen"), [
+    (128, (1, 1), 16, 300, 40),   # one row group, all waves on the chunks
+    (64, (1, 1), 33, 300, 70),    # a second row group of one row
+    (128, (2, 1), 32, 380, 70),   # 64 rows a wave, all waves on the chunks
+    (128, (3, 1), 32, 200, 70),   # two waves on the rows, the second half full
+    (64, (4, 1), 48, 390, 100),   # three turns of two waves
+    (96, (4, 2), 130, 260, 300),  # five turns of two waves, the last of four rows
+    (128, (8, 2), 72, 40, 100),   # five turns of four waves, two chunks
+    (128, (8, 1), 72, 1030, 150),  # nine turns, three windows of blocks
+])
+def test_rows_and_chunks_dealt_to_the_waves(cuda, dtype, d, heads, tq, nb, qlen):
+    _check(cuda, dtype, d, heads, tq, nb, qlen, 4 * nb - qlen - 3, 4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("d", "heads", "tq", "nb", "qlen"), [
     (256, (4, 1), 32, 64, 100),  # the mask alone from the owner kernel
     (256, (4, 1), 40, 70, 100),  # its second pass of rows
     (256, (2, 1), 40, 130, 90),  # fewer rows than a pass
