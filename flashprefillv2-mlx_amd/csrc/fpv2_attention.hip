@@ -1844,11 +1844,30 @@ extern "C" int64_t fpv2_sparse_attention_balanced_tiles(const fpv2_attn_params* 
   using namespace fpv2;
   if (!p || p->tile_q <= 0 || !balanced_ok(p, p->padded_query_length / p->tile_q)) return 0;
   const int64_t tiles = p->padded_query_length / p->tile_q;
-  // Up to half a turn of the chip every item can have two parts.  Measured at
-  // half a turn (D = 128, whole / parts): 499 steps a tile 338 / 238 us, 115
-  // steps 91 / 78 us, 96 steps 75 / 72 us, but 56 steps 48 / 52 us (the merge
-  // launch and the plan); at 0.6 turns 499 steps 358 / 369 us.
+  // up to half a turn of the chip every item can have two parts (D = 128, whole
+  // / parts: half a turn, 499 steps a tile 338 / 238 us; 0.6 turns 358 / 369 us)
   return balanced_items(p, tiles) * p->kv_heads * 2 <= workgroup_slots(p) ? tiles : 0;
+}
+
+extern "C" int64_t fpv2_sparse_attention_balanced_choice(const fpv2_attn_params* p, int dtype) {
+  using namespace fpv2;
+  const int64_t tiles = fpv2_sparse_attention_balanced_tiles(p);
+  if (tiles == 0 || p->query_length <= 0 || p->offset < 0) return 0;
+  // The longest walk the call can have: every block that starts at or before
+  // its last row.  Walks of up to kBalPart steps are not cut at all; longer ones
+  // have to win back the plan and the merge's launch, about 5 us, the more of
+  // them the fewer parts a tile can have, i.e. with the square of the call's
+  // share of the chip f.  Measured at f = 1/8, 1/4, 3/8, 1/2, the steps a tile
+  // from which parts are faster: bfloat16, D = 128: 36, 47, 66, 81; D = 96: 36,
+  // 52, 90, 105; D = 64: 40, 48, 85, 98; float16 (whose later parts walk
+  // online), D = 128: 40, 62, 107, 160; D = 256, both types: 36, 36, 44, 46.
+  // At f = 1/2 and D = 128, whole / parts: 48 steps 39 / 47 us, 96 steps 70 / 67 us,
+  // 192 steps 131 / 106 us.
+  const int64_t blocks = std::min(p->num_blocks, (p->offset + p->query_length - 1) / p->block_k + 1);
+  const double steps = static_cast<double>(blocks) * ((p->block_k + 31) / 32);
+  const double f = static_cast<double>(balanced_items(p, tiles) * p->kv_heads) / workgroup_slots(p);
+  const double slope = p->head_dim > 128 ? 64. : dtype == FPV2_F16 ? 512. : 256.;
+  return steps > kBalPart + slope * f * f ? tiles : 0;
 }
 
 extern "C" int64_t fpv2_sparse_attention_balanced_workspace_bytes(const fpv2_attn_params* p, int64_t tiles) {

@@ -45,6 +45,7 @@ EXPORTED_SYMBOLS = (
     "fpv2_sparse_attention_split",
     "fpv2_sparse_attention_split_static",
     "fpv2_sparse_attention_balanced_tiles",
+    "fpv2_sparse_attention_balanced_choice",
     "fpv2_sparse_attention_balanced_workspace_bytes",
     "fpv2_sparse_attention_balanced",
     # decoder-layer operations of the end-to-end harness (fpv2_decoder.h)
@@ -153,6 +154,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fpv2_sparse_attention_balanced_workspace_bytes.argtypes = [ctypes.POINTER(AttnParams), i64]
     lib.fpv2_sparse_attention_balanced_tiles.restype = i64
     lib.fpv2_sparse_attention_balanced_tiles.argtypes = [ctypes.POINTER(AttnParams)]
+    lib.fpv2_sparse_attention_balanced_choice.restype = i64
+    lib.fpv2_sparse_attention_balanced_choice.argtypes = [ctypes.POINTER(AttnParams), i32]
     lib.fpv2_sparse_attention_balanced.restype = ctypes.c_int
     lib.fpv2_sparse_attention_balanced.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i32,
                                                    ctypes.POINTER(AttnParams), i64, vp, i64, vp]

@@ -268,7 +268,7 @@ def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts
     kernel (``fpv2_sparse_attention_split``), with a workspace from the
     caching allocator.  ``balanced``: cut the walks into parts by their
     lengths instead, those of the last ``split_tiles`` tiles, or of all tiles
-    where the call has too few to fill the chip
+    where the call has too few to fill the chip and walks long enough to gain
     (``fpv2_sparse_attention_balanced``).
     """
     lib = _lib.load()
@@ -289,7 +289,8 @@ def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts
         pooled_head_stride=pooled_k.stride(0))
     with torch.cuda.device(device):
         if balanced:
-            split_tiles = lib.fpv2_sparse_attention_balanced_tiles(params) or split_tiles
+            split_tiles = lib.fpv2_sparse_attention_balanced_choice(
+                params, _lib.dtype_code(q.dtype)) or split_tiles
         if balanced and split_tiles:
             need = lib.fpv2_sparse_attention_balanced_workspace_bytes(params, split_tiles)
             if need < 0:

@@ -252,11 +252,17 @@ int fpv2_sparse_attention_split(const void* q, const void* k, const void* v,
                                 int64_t workspace_bytes, void* stream);
 
 /*
- * Query tiles of a call whose walks are worth cutting into parts on the
- * current device (fpv2_sparse_attention_balanced): all of them where whole
- * tiles would leave half of the chip idle, otherwise 0.
+ * Query tiles of a call whose walks can be cut into parts on the current
+ * device (fpv2_sparse_attention_balanced): all of them where whole tiles would
+ * leave half of the chip idle, otherwise 0.
  */
 int64_t fpv2_sparse_attention_balanced_tiles(const fpv2_attn_params* params);
+
+/*
+ * The same for inputs of `dtype`, and 0 where the longest walk that the call
+ * can have is too short to gain by being cut.
+ */
+int64_t fpv2_sparse_attention_balanced_choice(const fpv2_attn_params* params, int dtype);
 
 /*
  * Workspace bytes of fpv2_sparse_attention_balanced on the current device (0

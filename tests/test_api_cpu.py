@@ -351,6 +351,32 @@ def test_score_select_rejects_more_than_the_maximum_block_count():
     assert b"exceeds 8192" in lib.fpv2_last_error()
 
 
+@pytest.mark.parametrize(("dtype", "dim", "tiles", "shortest"), [
+    # (workgroup slots of 256 compute units: 512 up to head dim 128, else 256;
+    # the share of the chip f is tiles / slots, and parts need more than 32 +
+    # slope f^2 steps of 32 keys, slope 256, 512 in float16, 64 at head dim 256)
+    ("BF16", 128, 16, 33), ("BF16", 64, 64, 37), ("BF16", 128, 128, 49), ("BF16", 96, 256, 97),
+    ("F16", 128, 128, 65), ("F16", 64, 256, 161), ("F16", 256, 128, 49), ("BF16", 256, 64, 37),
+])
+def test_short_walks_are_not_cut_into_parts(dtype, dim, tiles, shortest):
+    """Calls whose longest walk is too short to gain by parts keep whole tiles."""
+    lib = _lib.load()
+
+    def choice(steps, n=tiles):
+        length, rows = 32 * steps, n
+        return lib.fpv2_sparse_attention_balanced_choice(_lib.AttnParams(
+            query_heads=128, kv_heads=1, head_dim=dim, padded_query_length=rows, query_length=rows,
+            out_rows=rows, key_length=length, num_blocks=steps, offset=length - rows, block_k=32,
+            tile_q=1, mean_correction=1, scale=0.1, q_head_stride=rows * dim, q_row_stride=dim,
+            k_head_stride=length * dim, k_row_stride=dim, v_head_stride=length * dim,
+            v_row_stride=dim, o_head_stride=rows * dim, o_row_stride=dim,
+            pooled_head_stride=steps * dim), getattr(_lib, dtype))
+
+    assert choice(shortest) == tiles and choice(shortest - 1) == 0
+    slots = 512 if dim <= 128 else 256
+    assert choice(4096, slots // 2) == slots // 2 and choice(4096, slots // 2 + 1) == 0
+
+
 def test_block_count_and_the_selection_limit():
     """Key blocks of a hook call, ``ceil(max(Lk, offset + Lq_pad) / block_k)``
     (``patch.py:123-131``), and the hook's routing rule: eligible calls with
