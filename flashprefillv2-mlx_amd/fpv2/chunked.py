@@ -167,6 +167,15 @@ class ChunkedPrefill:
                 return False
         if n == 0 or type(k) is not torch.Tensor or type(v) is not torch.Tensor:
             return False
+        # One workgroup copies and pools a block's rows one after the other;
+        # copies of their own spread over the chip.  Microseconds in one launch /
+        # apart at 1024-row blocks of head dim 256 (2^18 elements), 2048 new
+        # rows: 1 KV head 25 / 23, 8 heads 27 / 34; 2048-row blocks: 48 / 27 and 49 /
+        # 46; 512-row blocks 14 / 23.
+        rows = min(bk, old % bk + n)
+        if rows * self.head_dim >= 1 << 18 and (
+                rows * self.head_dim >= 1 << 19 or self.kv_heads * n < 16 * rows):
+            return False
         self.reserve(n)
         lib, device = _lib.load(), self.k.device
         with torch.cuda.device(device):

@@ -83,3 +83,31 @@ def test_refusals(cuda):
 
     assert call(2, 64) == _lib.FPV2_ERR_ARGUMENT
     assert call(1, 60) == _lib.FPV2_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize(("d", "block", "heads", "start", "n", "together"), [
+    (256, 1024, 1, 0, 1023, True), (256, 1024, 1, 0, 1024, False), (256, 1024, 1, 900, 2048, False),
+    (256, 1024, 8, 0, 2048, True), (256, 2048, 8, 0, 2048, False), (64, 4096, 1, 4000, 200, False),
+    (64, 4096, 1, 0, 200, True), (128, 128, 1, 70, 2048, True)])
+def test_large_blocks_are_appended_and_pooled_apart(cuda, d, block, heads, start, n, together):
+    """Blocks whose rows would pass through one workgroup slower than copies
+    and pooling apart; outputs and caches are the same either way."""
+    g = torch.Generator().manual_seed(n)
+    total = start + n
+    q, k, v = (torch.randn((heads, total, d), generator=g).to(torch.bfloat16).to(cuda)
+               for _ in range(3))
+    a, b = (ChunkedPrefill(heads, heads, d, total, device=cuda, min_tokens=1,
+                           config=FPV2Config(block_k=block, tile_q=128)) for _ in range(2))
+    calls = []
+    fused = a._append_pooled
+    a._append_pooled = lambda *args: calls.append(fused(*args)) or calls[-1]
+    if start:
+        for c in (a, b):
+            c.append(k[:, :start], v[:, :start])
+            c.attend(q[:, :start])
+    x = a.step(q[:, start:], k[:, start:], v[:, start:])
+    b.append(k[:, start:], v[:, start:])
+    y = b.attend(q[:, start:])
+    torch.cuda.synchronize()
+    assert calls == [together]
+    assert torch.equal(x, y) and _equal(a, b, total)
