@@ -344,7 +344,12 @@ class ChunkedPrefillRunner:
             for li in range(m.shape.layers):
                 x, delta = self._layer(li, x, delta, cos, sin)
         last = _add_rms_norm(x[-1:], delta[-1:], m.final_norm, m.shape.rms_eps)
-        return _row_logits(last[0], m.embed)
+        w = m.embed
+        if (w.stride(1) != 1 or w.stride(0) % 8 or w.stride(0) < w.shape[1] or w.data_ptr() % 16
+                or (w.requires_grad and torch.is_grad_enabled())):
+            # (rows that the kernel does not read in place, or a graph to keep)
+            return F.linear(last, w).float()[0]
+        return _row_logits(last[0], w)
 
 
 def measure(shape: DecoderShape, *, tokens: int, chunk: int, alpha: float, device,
