@@ -1736,7 +1736,7 @@ int score_select(const void* q, const void* pooled_k, int dtype, const fpv2_sele
   a.tq = p->tile_q;
   a.sink = p->sink_tokens;
   a.window = p->window_tokens;
-  a.last_n = p->last_n_blocks;
+  a.last_n = std::min(p->last_n_blocks, a.Nt);  // (the kernels keep it in 32 bits)
   a.scale = p->scale;
   a.alpha = p->alpha;
   a.q_hs = p->q_head_stride;

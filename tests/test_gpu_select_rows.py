@@ -210,3 +210,23 @@ def test_row_groups_over_2_gib_of_scores(cuda, dtype, heads, tq, length, nb):
     quarter = -(-length // 4 // tq) * tq
     _, _, ms4 = _scored(cuda, q[:, :quarter].contiguous(), pk, config)
     assert ms < 8 * ms4 + 0.2
+
+
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("last", [0, 3, 2 ** 31, 2 ** 33, 2 ** 63 - 1])
+def test_dense_tails_of_any_length(cuda, d, last):
+    """A dense tail past 32 bits covers every tile, in masks with and without
+    scores."""
+    g = torch.Generator().manual_seed(d)
+    q = torch.randn((2, 512, d), generator=g).to(torch.bfloat16).to(cuda)
+    pk = torch.randn((1, 130, d), generator=g).to(torch.bfloat16).to(cuda)
+    tiles = torch.arange(16)[:, None]
+    seen = torch.arange(130)[None] * 4 <= 8 + tiles * 32 + 31
+    for chunk in (None, 1):
+        # (no energy reaches ten times the largest)
+        config = FPV2Config(block_k=4, tile_q=32, alpha=10.0, sink_tokens=0, window_tokens=0,
+                            last_n_blocks=last, score_chunk_tiles=chunk)
+        sel, _ = block_scores_and_select(q, pk, scale=0.1, config=config, offset=8)
+        # (a window of 0 keeps the blocks that reach into the tile's first row on)
+        own = torch.arange(130)[None] * 4 + 4 > 8 + tiles * 32
+        assert torch.equal(sel[0].cpu(), seen & (own | (tiles >= 16 - last)))
