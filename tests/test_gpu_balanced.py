@@ -63,7 +63,7 @@ def _pad(x, multiple):
 
 
 # (queries, keys): one row; one tile; a last tile of one row; a short chunk of
-# a long prefix; a whole prompt; more items than workgroups of a head
+# a long prefix; a whole prompt; a chunk of many tiles
 @pytest.mark.parametrize(("n", "lk"), [(1, 5000), (32, 4096), (65, 3001), (300, 16000),
                                        (2048, 2048), (2100, 9000)])
 @pytest.mark.parametrize(("d", "dtype", "heads", "corr"), [
@@ -105,6 +105,38 @@ def test_only_the_last_tiles(cuda):
     torch.cuda.synchronize()
     assert torch.equal(outs[0][:, :-64], outs[1][:, :-64])
     _close(*outs)
+
+
+@pytest.mark.parametrize(("d", "tiles", "cut"), [
+    (64, 300, True),    # two items for some of the 256 threads that plan
+    (128, 430, True),   # most workgroups taken by whole items
+    (64, 1300, False),  # six items a thread, two past those it keeps
+    (256, 1300, False),  # three items for each of 512 threads
+])
+def test_plans_of_many_items(cuda, d, tiles, cut):
+    """More (tile, row chunk) items of a head than threads that plan, with
+    walks of 1 to 200 sub-tiles: parts where workgroups are left over, else
+    every item whole, and each item's rows from its own walk."""
+    g = torch.Generator(device=cuda).manual_seed(tiles)
+    n = 16 * tiles - 5
+    q = torch.randn((8, 16 * tiles, d), generator=g, device=cuda).to(torch.bfloat16)
+    q[:, n:] = 0
+    blocks = 16 * tiles // 128 + 60
+    k, v = (torch.randn((1, 128 * blocks, d), generator=g, device=cuda).to(torch.bfloat16)
+            for _ in range(2))
+    lk = 128 * blocks
+    config = FPV2Config(tile_q=16)
+    mask = torch.zeros((1, tiles, blocks), dtype=torch.bool, device=cuda)
+    length = torch.randint(1, 50, (tiles,), generator=g, device=cuda)
+    length[torch.randint(0, tiles, (tiles // 2,), generator=g, device=cuda)] = 1
+    mask[0] = torch.arange(blocks, device=cuda)[None] < length[:, None]
+    lists = compact_block_indices(mask, config=config, offset=lk - n, query_length=n, key_length=lk)
+    assert torch.equal(lists[1][0], length.to(torch.int32))
+    slots = 512 if d <= 128 else 256
+    assert (tiles < slots) == cut
+    whole, even = _both(q, k, v, pool_blocks(k), pool_blocks(v), lists, config, n, lk)
+    _close(whole, even)
+    assert torch.equal(whole, even) != cut
 
 
 def test_tiles_of_several_row_chunks_and_a_dense_tail(cuda):
