@@ -160,7 +160,8 @@ __device__ __forceinline__ int clampi(int x, int lo, int hi) {
 
 // ---------------------------------------------------------------------------
 // Balanced walk: bal_wgs workgroups per KV head (as many as the chip holds at
-// once) walk the head's (tile, row chunk) items in parts.  An item whose walk
+// once, or a few turns of them: balanced_turns) walk the head's (tile, row
+// chunk) items in parts.  An item whose walk
 // has `len` steps, taken from its list counts, becomes ceil(len / quantum)
 // equal parts, one workgroup each; the quantum is the smallest (in steps of
 // an eighth) for which the head's parts do not exceed its workgroups, and at
@@ -780,8 +781,8 @@ __global__ __launch_bounds__(WAVES * 64, ((D <= 128 || DS == 2) ? 2 : 1)) void s
   const int vm = GM::vmask(vrow);
   const uint32_t vbase = smem_lds + GM::TILE + (own + vrow) * ROWB + (((l16 & 3) >> 1) ^ vm) * 16 +
                          (l16 & 1) * 8 + dhalf * DT * 32;
-  // Walks whose ring stage is known at compile time (the 4-wave shape on
-  // whole tiles) read K and V at per-lane addresses computed once, with the
+  // Walks whose ring stage is known at compile time (the 4-wave shape, whole
+  // tiles and parts) read K and V at per-lane addresses computed once, with the
   // stage in the instruction's immediate offset: the XOR terms touch
   // address bits 4-7 only, which a stage offset (a multiple of the stage
   // size) leaves alone.
@@ -1817,24 +1818,71 @@ int64_t workgroup_slots(const fpv2_attn_params* p) {
 int64_t balanced_items(const fpv2_attn_params* p, int64_t tiles) {  // (tile, row chunk) items per KV head
   return tiles * ((p->query_heads / p->kv_heads * p->tile_q + kSplitRows - 1) / kSplitRows);
 }
-// workgroups per KV head: the chip's, and at least one per item
-int64_t balanced_wgs(const fpv2_attn_params* p, int64_t tiles) {
-  return std::max(workgroup_slots(p) / p->kv_heads, balanced_items(p, tiles));
+// The longest walk a tile can have, in steps: every block that starts at or
+// before its last row (the last tile's: the call's longest).
+int64_t longest_walk(const fpv2_attn_params* p, int64_t tile) {
+  const int64_t last = p->offset + std::min((tile + 1) * p->tile_q, p->query_length) - 1;
+  return std::min(p->num_blocks, last / p->block_k + 1) * ((p->block_k + 31) / 32);
+}
+int64_t longest_walk(const fpv2_attn_params* p) { return longest_walk(p, p->padded_query_length / p->tile_q - 1); }
+
+// Turns of the chip that the parts make: one for calls of few tiles.  For a
+// long dense tail, whose walks are known, an item has a whole number k of parts,
+// and where one turn of them leaves the chip idle, several turns of shorter
+// parts fill it: k is the one of the least time
+//   turns (average walk / k + c) + idle part of the last turn (shortest / k + c),
+// at least the longest part's, with c = 24 steps for a part's set-up and partial
+// and 10 % against more turns.  In float16 a longest part is added: a first part
+// whose reference fails walks again.  Whole sparse calls of 24576 keys, segments
+// of 128 steps / one turn / this: float16, 32 / 8 heads, 48 tail tiles (0.75
+// turns) 1664 / 2015 / 1513 us; D = 256, 16 / 4 heads, 71 tiles (1.1 turns)
+// 2151 / 2741 / 2024 us.
+constexpr int64_t kBalTurns = 6;
+int64_t balanced_turns(const fpv2_attn_params* p, int64_t tiles, bool f16) {
+  const int64_t slots = workgroup_slots(p), items = balanced_items(p, tiles) * p->kv_heads;
+  const int64_t all = p->padded_query_length / p->tile_q;
+  if (items == 0 || (tiles == all && 2 * items <= slots)) return 1;
+  const double f = static_cast<double>(items) / slots, c = 24.;
+  const double longest = static_cast<double>(longest_walk(p)), shortest = static_cast<double>(longest_walk(p, all - tiles));
+  const int64_t least = (items + slots - 1) / slots;  // of whole items
+  int64_t turns = least;
+  double best = 0.;
+  for (int64_t n = least; n == least || n <= kBalTurns; ++n) {
+    const double k = static_cast<double>(n * slots / items);
+    if (n > least && longest < kBalPart * k) break;
+    const double full = f * k, idle = __builtin_ceil(full) - full;
+    const double t = std::max(full * ((longest + shortest) / 2. / k + c) + idle * (shortest / k + c), longest / k + c) +
+                     (f16 ? longest / k : 0.);
+    if (n == least || t < 0.9 * best) {
+      best = t;
+      turns = n;
+    }
+  }
+  return turns;
+}
+// workgroups per KV head, at least one per item
+int64_t balanced_wgs(const fpv2_attn_params* p, int64_t tiles, bool f16) {
+  return std::max(balanced_turns(p, tiles, f16) * workgroup_slots(p) / p->kv_heads, balanced_items(p, tiles));
+}
+// (the caller's workspace serves both types)
+int64_t balanced_wgs_max(const fpv2_attn_params* p, int64_t tiles) {
+  return std::max(balanced_wgs(p, tiles, false), balanced_wgs(p, tiles, true));
 }
 int64_t balanced_bytes(const fpv2_attn_params* p, int64_t tiles) {
-  return p->kv_heads * (balanced_wgs(p, tiles) * kSplitRows * (p->head_dim + 2) * 4 +
+  return p->kv_heads * (balanced_wgs_max(p, tiles) * kSplitRows * (p->head_dim + 2) * 4 +
                         balanced_items(p, tiles) * static_cast<int64_t>(sizeof(BalCut)));
 }
 // Whether the parameters are complete and the sums over a head's items and
 // the grid fit 32 bits.
 bool balanced_ok(const fpv2_attn_params* p, int64_t tiles) {
   if (!p || p->tile_q <= 0 || p->padded_query_length <= 0 || p->kv_heads <= 0 || p->query_heads <= 0 ||
-      p->query_heads % p->kv_heads || p->block_k <= 0 || p->num_blocks <= 0 || p->head_dim <= 0)
+      p->query_heads % p->kv_heads || p->block_k <= 0 || p->num_blocks <= 0 || p->head_dim <= 0 ||
+      p->query_length <= 0 || p->offset < 0)
     return false;
   if (tiles < 0 || tiles > p->padded_query_length / p->tile_q) return false;
   const int64_t steps = p->num_blocks * ((p->block_k + 31) / 32 + 1) + 1;
   return steps < (1LL << 31) && balanced_items(p, tiles) <= ((1LL << 31) - 1) / steps &&
-         p->kv_heads <= 65535 && balanced_wgs(p, tiles) * p->kv_heads <= 0x7fffffffLL / 16;
+         p->kv_heads <= 65535 && balanced_wgs_max(p, tiles) * p->kv_heads <= 0x7fffffffLL / 16;
 }
 
 }  // namespace
@@ -1852,22 +1900,19 @@ extern "C" int64_t fpv2_sparse_attention_balanced_tiles(const fpv2_attn_params* 
 extern "C" int64_t fpv2_sparse_attention_balanced_choice(const fpv2_attn_params* p, int dtype) {
   using namespace fpv2;
   const int64_t tiles = fpv2_sparse_attention_balanced_tiles(p);
-  if (tiles == 0 || p->query_length <= 0 || p->offset < 0) return 0;
-  // The longest walk the call can have: every block that starts at or before
-  // its last row.  Walks of up to kBalPart steps are not cut at all; longer ones
-  // have to win back the plan and the merge's launch, about 5 us, the more of
-  // them the fewer parts a tile can have, i.e. with the square of the call's
+  if (tiles == 0) return 0;
+  // Walks of up to kBalPart steps are not cut at all; longer ones have to win
+  // back the plan and the merge's launch, about 5 us, the more of them the fewer
+  // parts a tile can have, i.e. with the square of the call's
   // share of the chip f.  Measured at f = 1/8, 1/4, 3/8, 1/2, the steps a tile
   // from which parts are faster: bfloat16, D = 128: 36, 47, 66, 81; D = 96: 36,
   // 52, 90, 105; D = 64: 40, 48, 85, 98; float16 (whose later parts walk
   // online), D = 128: 40, 62, 107, 160; D = 256, both types: 36, 36, 44, 46.
   // At f = 1/2 and D = 128, whole / parts: 48 steps 39 / 47 us, 96 steps 70 / 67 us,
   // 192 steps 131 / 106 us.
-  const int64_t blocks = std::min(p->num_blocks, (p->offset + p->query_length - 1) / p->block_k + 1);
-  const double steps = static_cast<double>(blocks) * ((p->block_k + 31) / 32);
   const double f = static_cast<double>(balanced_items(p, tiles) * p->kv_heads) / workgroup_slots(p);
   const double slope = p->head_dim > 128 ? 64. : dtype == FPV2_F16 ? 512. : 256.;
-  return steps > kBalPart + slope * f * f ? tiles : 0;
+  return static_cast<double>(longest_walk(p)) > kBalPart + slope * f * f ? tiles : 0;
 }
 
 extern "C" int64_t fpv2_sparse_attention_balanced_workspace_bytes(const fpv2_attn_params* p, int64_t tiles) {
@@ -1898,7 +1943,7 @@ extern "C" int fpv2_sparse_attention_balanced(const void* q, const void* k, cons
                   static_cast<long long>(need));
     if (reinterpret_cast<uintptr_t>(workspace) % 16)
       return fail(FPV2_ERR_ARGUMENT, "sparse_attention_balanced: workspace must be 16-byte aligned");
-    const int64_t wgs = balanced_wgs(p, tiles);
+    const int64_t wgs = balanced_wgs(p, tiles, dtype == FPV2_F16);
     a.split_tiles = static_cast<int>(tiles);
     a.bal_wgs = static_cast<int>(wgs);
     a.ws_o = static_cast<float*>(workspace);

@@ -377,6 +377,27 @@ def test_short_walks_are_not_cut_into_parts(dtype, dim, tiles, shortest):
     assert choice(4096, slots // 2) == slots // 2 and choice(4096, slots // 2 + 1) == 0
 
 
+@pytest.mark.parametrize(("dim", "tiles", "turns"), [
+    (128, 96, 1),     # 3/16 of a turn of the 512 slots, one turn of parts
+    (128, 384, 3),    # three quarters of a turn: a whole turn of uncut walks would idle
+    (256, 288, 2),    # more than one turn of 256: a second, nearly empty one
+    (128, 1024, 2),   # two whole turns
+])
+def test_long_dense_tails_fill_the_chip(dim, tiles, turns):
+    """Workgroups for a dense tail (from the workspace): several turns of parts
+    where one of whole walks would leave much of the chip idle."""
+    lib = _lib.load()
+    p = _lib.AttnParams(
+        query_heads=128, kv_heads=1, head_dim=dim, padded_query_length=4096, query_length=4096,
+        out_rows=4096, key_length=65536, num_blocks=512, offset=61440, block_k=128, tile_q=1,
+        mean_correction=1, scale=0.1, q_head_stride=4096 * dim, q_row_stride=dim,
+        k_head_stride=65536 * dim, k_row_stride=dim, v_head_stride=65536 * dim, v_row_stride=dim,
+        o_head_stride=4096 * dim, o_row_stride=dim, pooled_head_stride=512 * dim)
+    need = lib.fpv2_sparse_attention_balanced_workspace_bytes(p, tiles)
+    slots = 512 if dim <= 128 else 256
+    assert need >= turns * slots * 128 * (dim + 2) * 4
+
+
 def test_block_count_and_the_selection_limit():
     """Key blocks of a hook call, ``ceil(max(Lk, offset + Lq_pad) / block_k)``
     (``patch.py:123-131``), and the hook's routing rule: eligible calls with

@@ -107,16 +107,17 @@ def test_only_the_last_tiles(cuda):
     _close(*outs)
 
 
-@pytest.mark.parametrize(("d", "tiles", "cut"), [
-    (64, 300, True),    # two items for some of the 256 threads that plan
-    (128, 430, True),   # most workgroups taken by whole items
-    (64, 1300, False),  # six items a thread, two past those it keeps
-    (256, 1300, False),  # three items for each of 512 threads
+@pytest.mark.parametrize(("d", "tiles"), [
+    (64, 300),    # two items for some of the 256 threads that plan, four turns
+    (128, 430),
+    (64, 1300),   # six items a thread, two past those it keeps
+    (256, 1300),  # three items for each of 512 threads
+    (96, 3300),   # more turns than parts would be cut for
 ])
-def test_plans_of_many_items(cuda, d, tiles, cut):
+def test_plans_of_many_items(cuda, d, tiles):
     """More (tile, row chunk) items of a head than threads that plan, with
-    walks of 1 to 200 sub-tiles: parts where workgroups are left over, else
-    every item whole, and each item's rows from its own walk."""
+    walks of 1 to 200 sub-tiles, some of them whole and some in parts: each
+    item's rows come from its own walk."""
     g = torch.Generator(device=cuda).manual_seed(tiles)
     n = 16 * tiles - 5
     q = torch.randn((8, 16 * tiles, d), generator=g, device=cuda).to(torch.bfloat16)
@@ -132,11 +133,9 @@ def test_plans_of_many_items(cuda, d, tiles, cut):
     mask[0] = torch.arange(blocks, device=cuda)[None] < length[:, None]
     lists = compact_block_indices(mask, config=config, offset=lk - n, query_length=n, key_length=lk)
     assert torch.equal(lists[1][0], length.to(torch.int32))
-    slots = 512 if d <= 128 else 256
-    assert (tiles < slots) == cut
     whole, even = _both(q, k, v, pool_blocks(k), pool_blocks(v), lists, config, n, lk)
     _close(whole, even)
-    assert torch.equal(whole, even) != cut
+    assert not torch.equal(whole, even)
 
 
 def test_tiles_of_several_row_chunks_and_a_dense_tail(cuda):
