@@ -250,7 +250,9 @@ def _pooled_ready(pooled_k: torch.Tensor, pooled_v: torch.Tensor):
 
 
 # Sub-tiles (32 keys each) per segment of a split tile: 4096 keys, about
-# the walk of a typical tile of a sparse long-context layer.
+# the walk of a typical tile of a sparse long-context layer.  (The hook's dense
+# tail is cut by the balanced walk once it is longer than two of them; fixed
+# segments are kept for the split entry points, which may not plan on the device.)
 SPLIT_SEG_STEPS = 128
 
 
@@ -266,7 +268,8 @@ def _launch_attention(q, k, v, pooled_k, pooled_v, selected_ids, selected_counts
     are never read.  ``split_tiles``: run the last ``split_tiles`` query
     tiles as key-range segments of ``seg_steps`` sub-tiles, merged after the
     kernel (``fpv2_sparse_attention_split``), with a workspace from the
-    caching allocator.  ``balanced``: cut the walks into parts by their
+    caching allocator (no caller of the package asks for it without
+    ``balanced``).  ``balanced``: cut the walks into parts by their
     lengths instead, those of the last ``split_tiles`` tiles, or of all tiles
     where the call has too few to fill the chip and walks long enough to gain
     (``fpv2_sparse_attention_balanced``).

@@ -198,7 +198,8 @@ def block_scores_and_select(
                             padded_length=padded_length,
                             key_length=num_blocks * config.block_k)
     with torch.cuda.device(device):
-        # (a mask of 16-bit inputs alone takes the streaming path, which has no use for it)
+        # (16-bit masks alone take the streaming or owner kernel, which have no use for it;
+        # at head dim 256 and few blocks the row path, with whole tiles)
         rows = scores is not None or dtype == torch.float32 or not scale > 0
         need = lib.fpv2_score_select_workspace_bytes(params) if rows else 0
         if need:

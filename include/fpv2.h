@@ -272,13 +272,13 @@ int64_t fpv2_sparse_attention_balanced_workspace_bytes(const fpv2_attn_params* p
 
 /*
  * fpv2_sparse_attention with the walks of the last `tiles` query tiles cut
- * into parts of similar length, as many as the chip holds workgroups; a
- * second kernel adds a tile's partials.  For calls with few tiles (a short
+ * into parts of similar length, as many as the chip holds workgroups (a few
+ * times as many for a long dense tail); a second kernel adds a tile's partials.  For calls with few tiles (a short
  * chunk of queries, few KV heads, one GPU's share of a layer) and for a dense
  * tail among sparse tiles.  The parts follow from the list counts, on the
  * device.  The result equals fpv2_sparse_attention's up to
- * float32 summation order, the other tiles' rows bit for bit; it is
- * deterministic.  workspace: at least the bytes above, 16-byte aligned, owned
+ * float32 summation order (NaN and infinite where that is), the other tiles'
+ * rows bit for bit; it is deterministic.  workspace: at least the bytes above, 16-byte aligned, owned
  * by the caller (no contents are kept between calls); calls that share a
  * workspace on different streams race.  No counterpart in the reference
  * (fpv2/kernel.py:248-325: one threadgroup per query tile).

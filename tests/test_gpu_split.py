@@ -137,10 +137,10 @@ def test_split_tiles_of_several_row_chunks(cuda):
 
 
 def test_hook_splits_a_long_dense_tail(cuda):
-    """The hook splits its dense tail once the walk exceeds two segments of
-    128 sub-tiles: at 16384 keys with the contrast generator, the last two
-    tiles run as 4 segments each; outputs equal the unsplit run up to
-    float32 summation order, and the tail rows match the oracle."""
+    """The hook cuts its dense tail into parts once the walk exceeds 256
+    sub-tiles: at 16384 keys with the contrast generator, the last two tiles;
+    the other tiles' rows are the whole run's bit for bit, the tail's equal up
+    to float32 summation order and match the oracle."""
     from fpv2.patch import _fpv2_sdpa
     seq = 16384
     q, k, v = baseline_qkv(seq, planted=3.0 * 128 ** 0.5, heavy_fraction=0.06, seed=4,
